@@ -244,7 +244,8 @@ void launchHashEncodeKernel(MLPGridOptions* opt, half* d_hashtable, const float*
 {
     guarded("launchHashEncodeKernel", [&] {
         const graft::GridMeta m = meta(opt);
-        graft::hash_encode(m, d_hashtable, d_inputs, inputStride, d_enc_out, batchSize, stream);
+        graft::hash_encode(m, d_hashtable, d_inputs, inputStride, d_enc_out, batchSize, stream, nullptr,
+                           &graft::stream_encode_scratch(stream));
     });
 }
 

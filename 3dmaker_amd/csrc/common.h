@@ -6,6 +6,7 @@
 #include <hip/hip_fp16.h>
 
 #include <cstdint>
+#include <mutex>
 #include <stdexcept>
 #include <string>
 
@@ -91,16 +92,27 @@ public:
     Workspace(const Workspace&) = delete;
     Workspace& operator=(const Workspace&) = delete;
     void* get(size_t bytes);
+    // At least `bytes` for work on stream s, or nullptr (what is held stays)
+    // when the stream is being captured (a graph would keep an address that a
+    // later call may free), is hipStreamPerThread or the memory cannot be had:
+    // for callers that have another way.  mutex() is theirs to hold while they
+    // enqueue what uses it.
+    void* try_get(size_t bytes, hipStream_t s);
+    std::mutex& mutex() { return mu_; }
     size_t size() const { return bytes_; }
 
 private:
     void* p_ = nullptr;
     size_t bytes_ = 0;
+    std::mutex mu_;
 };
 
 // The workspace of (current device, stream), for callers without an owner of
 // their own (the extern "C" launchers); kept until the process ends.
 Workspace& stream_workspace(hipStream_t s);
+// Likewise for level-major encodings (a buffer of its own: they live beside
+// what stream_workspace holds).
+Workspace& stream_encode_scratch(hipStream_t s);
 
 int num_cus();
 

@@ -70,48 +70,87 @@ __device__ __forceinline__ void stage_meta(const GridKernelArgs& a, float* ss, i
 }
 
 // gfx950 dispatches workgroup i to XCD i mod 8, and each XCD has its own 4 MB
-// L2.  The encode gives each XCD its own levels, so that its L2 holds only
-// those levels' fp16 tables (2 MiB per hashed level at T = 2^19) instead of
-// cycling all 32 MiB through every L2: levels are dealt to XCDs in snake
-// order, l -> l mod 8 for even l / 8 and 7 - l mod 8 for odd, which pairs
-// level l with level 15 - l (a small dense level with a hashed one).
+// L2.  The encode gives each XCD its own levels, dealt in snake order, l -> l
+// mod 8 for even l / 8 and 7 - l mod 8 for odd, which pairs level l with level
+// 15 - l (a small dense level with a hashed one).
 constexpr int kXcds = 8;
+constexpr int kEncodeTile = 256;       // samples of one workgroup
+constexpr int kEncodeTiles = 1 << 16;  // sample tiles of one launch: more are looped over
 
-// Each workgroup encodes, for every sample of its stride, the levels of its
-// XCD, 16 k + x and 16 k + 15 - x; both are computed unconditionally (an
-// out-of-range level reads level 0 and is not stored) so that their gathers
-// are in flight together.  Output: PLANAR, enc[l][plane] feature pairs; else
-// row-major enc[n][2L].
-template <bool PLANAR>
-__global__ __launch_bounds__(256) void hash_encode_kernel(const GridKernelArgs a, const float* __restrict__ pos,
-                                                          const _Float16* __restrict__ table,
-                                                          _Float16* __restrict__ enc, int plane)
+// Scattered points (SCATTERED): one workgroup encodes one level for one tile
+// of 256 samples.  Workgroups of an XCD are ordered level by level, its finest
+// first, so that the XCD works on one fp16 table at a time (2 MiB at T = 2^19,
+// half of its L2).  What bounds it is the lines the corner gathers bring from
+// the L2 into a CU's L1: a 128-byte line takes 1.8 to 2.4 cycles of a CU
+// (measured with random gathers of 4, 8 and 16 bytes, which all cost the
+// same), 64 lines per sample at 16 levels: 257 us for 2^20.
+// Samples in ray or cell order (!SCATTERED) share most lines of the coarse
+// levels with their neighbours; there a tile's workgroup takes the XCD's two
+// levels of each 16 together, one position load and twice the gathers in
+// flight.
+// Measured at T = 2^19, b = 1.3819, level-major output, SCATTERED / not, and
+// 2,048 looping workgroups with two levels per thread and 4-byte gathers
+// before: 2^20 uniform points 285 / 350, before 354 us; 2^18 uniform 79 / 93,
+// before 94 us; 2^18 ray-ordered 48.6 / 46.4, before 48.6 us; 2^20 ray-ordered
+// 171 / 166, before 174 us.
+// Output: PLANAR, enc[l][plane] feature pairs; else row-major enc[n][2L].
+template <bool PLANAR, bool SCATTERED>
+__global__ __launch_bounds__(kEncodeTile) void hash_encode_kernel(const GridKernelArgs a,
+                                                                  const float* __restrict__ pos,
+                                                                  const _Float16* __restrict__ table,
+                                                                  _Float16* __restrict__ enc, int plane, int tiles)
 {
-    __shared__ float ss[kMaxLevels];
-    __shared__ int sr[kMaxLevels];
-    stage_meta(a, ss, sr);
-    const uint32_t mask = (uint32_t)a.T - 1u;
     const int N = a.d_n ? min((int)*a.d_n, a.N) : a.N;
-    const int x = blockIdx.x % kXcds, nb = gridDim.x / kXcds;
+    const int x = blockIdx.x % kXcds, item = blockIdx.x / kXcds;
+    const int groups = (a.L + kXcds - 1) / kXcds;
+    const int k = SCATTERED ? item / tiles : 0;
+    const uint32_t mask = (uint32_t)a.T - 1u;
     const int D = 2 * a.L;
-    for (int n = (blockIdx.x / kXcds) * blockDim.x + threadIdx.x; n < N; n += nb * blockDim.x) {
+    for (long long n = (long long)(item - k * tiles) * kEncodeTile + threadIdx.x; n < N;
+         n += (long long)tiles * kEncodeTile) {
         const float* pp = pos + (size_t)n * a.pos_stride;
         const float px = pp[0], py = pp[1], pz = pp[2];
-        for (int base = 0; base < a.L; base += 2 * kXcds) {
-            const int la = base + x, lb = base + 2 * kXcds - 1 - x;
-            const bool va = la < a.L, vb = lb < a.L;
-            const int ca = va ? la : 0, cb = vb ? lb : 0;
-            const float2 ea = encode_level(px, py, pz, ss[ca], sr[ca], ca < a.dense_start, mask,
-                                           table + (size_t)ca * a.T * 2);
-            const float2 eb = encode_level(px, py, pz, ss[cb], sr[cb], cb < a.dense_start, mask,
-                                           table + (size_t)cb * a.T * 2);
-            const h2 ha{to_h(ea.x), to_h(ea.y)}, hb{to_h(eb.x), to_h(eb.y)};
-            if constexpr (PLANAR) {
-                if (va) *reinterpret_cast<h2*>(enc + ((size_t)la * plane + n) * 2) = ha;
-                if (vb) *reinterpret_cast<h2*>(enc + ((size_t)lb * plane + n) * 2) = hb;
+        auto level = [&](int g) {
+            const int l = kXcds * g + ((g & 1) ? kXcds - 1 - x : x);
+            if (l >= a.L) return;
+            const float2 e = encode_level(px, py, pz, a.scale[l], a.res[l], l < a.dense_start, mask,
+                                          table + (size_t)l * a.T * 2);
+            const size_t at = PLANAR ? ((size_t)l * plane + n) * 2 : (size_t)n * D + 2 * l;
+            *reinterpret_cast<h2*>(enc + at) = h2{to_h(e.x), to_h(e.y)};
+        };
+        if constexpr (SCATTERED) {
+            level(groups - 1 - k);
+        } else {
+            for (int g = groups - 1; g >= 0; g -= 2) {
+                level(g);
+                if (g > 0) level(g - 1);
+            }
+        }
+    }
+}
+
+// Level-major encodings to rows [n][2L]: four lanes per sample, four levels a
+// lane at a time, so that a wave reads 64 contiguous bytes per level and
+// stores whole rows (16 bytes per lane where rows allow it).  2^18 samples of
+// 16 levels: 8 us.
+__global__ __launch_bounds__(256) void encode_rows_kernel(const _Float16* __restrict__ planar, int plane, int L, int N,
+                                                          _Float16* __restrict__ enc)
+{
+    typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+    const int sub = threadIdx.x & 3;
+    for (long long n = (long long)blockIdx.x * 64 + (threadIdx.x >> 2); n < N; n += (long long)gridDim.x * 64) {
+        for (int l = 4 * sub; l < L; l += 16) {
+            h2 v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (l + j < L) v[j] = *reinterpret_cast<const h2*>(planar + ((size_t)(l + j) * plane + n) * 2);
+            h2* dst = reinterpret_cast<h2*>(enc + (size_t)n * 2 * L + 2 * l);
+            if (l + 4 <= L && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
+                *reinterpret_cast<h8*>(dst) = h8{v[0].x, v[0].y, v[1].x, v[1].y, v[2].x, v[2].y, v[3].x, v[3].y};
             } else {
-                if (va) *reinterpret_cast<h2*>(enc + (size_t)n * D + 2 * la) = ha;
-                if (vb) *reinterpret_cast<h2*>(enc + (size_t)n * D + 2 * lb) = hb;
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (l + j < L) dst[j] = v[j];
             }
         }
     }
@@ -201,38 +240,57 @@ GridKernelArgs grid_args(const GridMeta& m, int N, int pos_stride)
     return a;
 }
 
-// kXcds workgroups per 256 samples, at most 256 per XCD; at least one per XCD
-// so that every level has a workgroup.
-int encode_blocks(int N)
+template <bool PLANAR, bool SCATTERED>
+void launch_encode(const GridMeta& m, const __half* table, const float* pos, int pos_stride, __half* enc, int plane,
+                   int N, hipStream_t stream, const uint32_t* d_n)
 {
-    return kXcds * std::max(1, std::min((N + 255) / 256, 256));
+    GridKernelArgs a = grid_args(m, N, pos_stride);
+    a.d_n = d_n;
+    const int tiles = std::min((N - 1) / kEncodeTile + 1, kEncodeTiles);
+    const int groups = (m.numLevels + kXcds - 1) / kXcds;
+    hipLaunchKernelGGL((hash_encode_kernel<PLANAR, SCATTERED>), dim3(kXcds * tiles * (SCATTERED ? groups : 1)),
+                       dim3(kEncodeTile), 0, stream, a, pos, reinterpret_cast<const _Float16*>(table),
+                       reinterpret_cast<_Float16*>(enc), plane, tiles);
+    GRAFT_LAUNCH_CHECK();
 }
 
 }  // namespace
 
+// Row-major output costs the encode a partial line per level and sample; from
+// kRowsFromPlanar samples on, level-major encodings in `scratch` and a pass
+// that turns them into rows are the faster way.  The two launches are
+// enqueued under the scratch's lock, so that calls of several threads on one
+// stream do not come between each other's.
 void hash_encode(const GridMeta& m, const __half* table, const float* pos, int pos_stride,
-                 __half* enc, int N, hipStream_t stream, const uint32_t* d_n)
+                 __half* enc, int N, hipStream_t stream, const uint32_t* d_n, Workspace* scratch)
 {
     if (N <= 0) return;
     if (pos_stride < 3) throw std::runtime_error("hash encode: position stride must be >= 3");
-    GridKernelArgs a = grid_args(m, N, pos_stride);
-    a.d_n = d_n;
-    hipLaunchKernelGGL(hash_encode_kernel<false>, dim3(encode_blocks(N)), dim3(256), 0, stream, a, pos,
-                       reinterpret_cast<const _Float16*>(table), reinterpret_cast<_Float16*>(enc), 0);
-    GRAFT_LAUNCH_CHECK();
+    constexpr int kRowsFromPlanar = 1 << 15;
+    if (scratch && !d_n && N >= kRowsFromPlanar) {
+        std::lock_guard<std::mutex> lk(scratch->mutex());
+        if (void* planar = scratch->try_get((size_t)N * m.numLevels * 2 * sizeof(__half), stream)) {
+            launch_encode<true, true>(m, table, pos, pos_stride, static_cast<__half*>(planar), N, N, stream, nullptr);
+            hipLaunchKernelGGL(encode_rows_kernel, dim3(std::min((N + 63) / 64, 1 << 20)), dim3(256), 0, stream,
+                               static_cast<const _Float16*>(planar), N, m.numLevels, N,
+                               reinterpret_cast<_Float16*>(enc));
+            GRAFT_LAUNCH_CHECK();
+            return;
+        }
+    }
+    launch_encode<false, true>(m, table, pos, pos_stride, enc, 0, N, stream, d_n);
 }
 
 void hash_encode_planar(const GridMeta& m, const __half* table, const float* pos, int pos_stride,
-                        __half* enc, int plane, int N, hipStream_t stream, const uint32_t* d_n)
+                        __half* enc, int plane, int N, hipStream_t stream, const uint32_t* d_n, bool scattered)
 {
     if (N <= 0) return;
     if (pos_stride < 3) throw std::runtime_error("hash encode: position stride must be >= 3");
     if (plane < N) throw std::runtime_error("hash encode: plane stride below the sample count");
-    GridKernelArgs a = grid_args(m, N, pos_stride);
-    a.d_n = d_n;
-    hipLaunchKernelGGL(hash_encode_kernel<true>, dim3(encode_blocks(N)), dim3(256), 0, stream, a, pos,
-                       reinterpret_cast<const _Float16*>(table), reinterpret_cast<_Float16*>(enc), plane);
-    GRAFT_LAUNCH_CHECK();
+    if (scattered)
+        launch_encode<true, true>(m, table, pos, pos_stride, enc, plane, N, stream, d_n);
+    else
+        launch_encode<true, false>(m, table, pos, pos_stride, enc, plane, N, stream, d_n);
 }
 
 void hash_scatter_atomic(const GridMeta& m, const __half* denc, const float* pos, int pos_stride,
@@ -292,6 +350,38 @@ void* Workspace::get(size_t bytes)
         bytes_ = nb;
     }
     return p_;
+}
+
+void* Workspace::try_get(size_t bytes, hipStream_t s)
+{
+    // hipStreamPerThread names another stream in every thread
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (s == hipStreamPerThread || hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (bytes <= bytes_) return p_;
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (p_) (void)hipFree(p_);
+    p_ = p;
+    bytes_ = bytes;
+    return p_;
+}
+
+Workspace& stream_encode_scratch(hipStream_t s)
+{
+    int dev = 0;
+    GRAFT_HIP_CHECK(hipGetDevice(&dev));
+    std::lock_guard<std::mutex> lk(g_ws_mu);
+    static std::map<std::pair<int, hipStream_t>, std::unique_ptr<Workspace>>* cache =
+        new std::map<std::pair<int, hipStream_t>, std::unique_ptr<Workspace>>();  // outlives static destructors
+    auto& w = (*cache)[{dev, s}];
+    if (!w) w.reset(new Workspace());
+    return *w;
 }
 
 Workspace& stream_workspace(hipStream_t s)
