@@ -158,6 +158,7 @@ void launchNetworkFusionHashTableKernel(MLPGridOptions* opt, half* d_hashtable, 
         in.pos_stride = 4;
         in.table = d_hashtable;
         in.meta = &m;
+        in.scratch = &graft::stream_encode_scratch(stream);
         graft::mlp_forward(shape(opt), in, W, B, nullptr, d_outputs, batchSize, OUT_ACT_NONE, stream);
     });
 }
@@ -173,6 +174,7 @@ void launchNetworkFusionHashTableGradKernel(MLPGridOptions* opt, half* d_hashtab
         in.pos_stride = 4;
         in.table = d_hashtable;
         in.meta = &m;
+        in.scratch = &graft::stream_encode_scratch(stream);
         graft::mlp_forward(shape(opt), in, W, B, acts, d_outputs, batchSize, OUT_ACT_NONE, stream);
     });
 }

@@ -6,9 +6,12 @@
 #include <hip/hip_fp16.h>
 
 #include <cstdint>
+#include <map>
+#include <memory>
 #include <mutex>
 #include <stdexcept>
 #include <string>
+#include <utility>
 
 #define GRAFT_HIP_CHECK(expr)                                                          \
     do {                                                                               \
@@ -110,8 +113,18 @@ private:
 // The workspace of (current device, stream), for callers without an owner of
 // their own (the extern "C" launchers); kept until the process ends.
 Workspace& stream_workspace(hipStream_t s);
-// Likewise for level-major encodings (a buffer of its own: they live beside
-// what stream_workspace holds).
+// One Workspace per (device, stream) a caller works on: calls of several
+// threads and streams each find their stream's, and all go with the owner.
+class StreamScratch {
+public:
+    Workspace& of(hipStream_t s);
+
+private:
+    std::mutex mu_;
+    std::map<std::pair<int, hipStream_t>, std::unique_ptr<Workspace>> ws_;
+};
+
+// That of the extern "C" launchers for level-major encodings.
 Workspace& stream_encode_scratch(hipStream_t s);
 
 int num_cus();

@@ -372,16 +372,20 @@ void* Workspace::try_get(size_t bytes, hipStream_t s)
     return p_;
 }
 
-Workspace& stream_encode_scratch(hipStream_t s)
+Workspace& StreamScratch::of(hipStream_t s)
 {
     int dev = 0;
     GRAFT_HIP_CHECK(hipGetDevice(&dev));
-    std::lock_guard<std::mutex> lk(g_ws_mu);
-    static std::map<std::pair<int, hipStream_t>, std::unique_ptr<Workspace>>* cache =
-        new std::map<std::pair<int, hipStream_t>, std::unique_ptr<Workspace>>();  // outlives static destructors
-    auto& w = (*cache)[{dev, s}];
+    std::lock_guard<std::mutex> lk(mu_);
+    auto& w = ws_[{dev, s}];
     if (!w) w.reset(new Workspace());
     return *w;
+}
+
+Workspace& stream_encode_scratch(hipStream_t s)
+{
+    static StreamScratch* all = new StreamScratch();  // outlives static destructors
+    return all->of(s);
 }
 
 Workspace& stream_workspace(hipStream_t s)

@@ -25,7 +25,16 @@ struct FwdInput {
     int pos_stride = 4;
     const __half* table = nullptr;
     const GridMeta* meta = nullptr;
+    // For the shapes mlp_forward_wide() names, else ignored: rows of x_dim
+    // features (0: in; the rest of the input is zero), the first user_dim
+    // outputs (0: out) also stored as rows at user (nullable), and (hash grid)
+    // room for level-major encodings of large batches (nullable).
+    int x_dim = 0;
+    float* user = nullptr;
+    int user_dim = 0;
+    Workspace* scratch = nullptr;
 };
+bool mlp_forward_wide(const MlpShape& s);
 
 // W, B, acts are DEVICE arrays of per-layer device pointers.  acts == nullptr
 // selects the inference kernel (no activation saves).

@@ -20,6 +20,7 @@
 #include "mlp.h"
 
 #include "hash_encode.h"
+#include "mlp32.h"
 #include "mlp_device.h"
 
 #include <algorithm>
@@ -669,12 +670,18 @@ static void fill_layer_offsets(const MlpShape& s, bool transposed, int* frag_off
 }
 
 
+bool mlp_forward_wide(const MlpShape& s) { return mlp32_forward_supported(s); }
+
 void mlp_forward(const MlpShape& s, const FwdInput& in, const __half* const* W,
                  const float* const* B, __half* const* acts, float* out, int N, int out_act,
                  hipStream_t stream, const uint32_t* d_n)
 {
     s.validate();
     if (N <= 0) return;
+    if (mlp32_forward_supported(s)) {
+        mlp32_forward(s, in, W, B, acts, out, N, out_act, stream, d_n);
+        return;
+    }
     FwdParams p{};
     p.pos = in.pos;
     p.pos_stride = in.pos_stride;

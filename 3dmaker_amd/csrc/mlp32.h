@@ -1,0 +1,18 @@
+// The 16x16x32 MFMA kernels of the fused MLP (mlp32.hip), behind mlp_forward
+// and mlp_backward for the shapes they take.
+#pragma once
+
+#include "mlp.h"
+
+namespace graft {
+
+// Samples from which the hash-grid forward encodes in a launch of its own, and
+// the samples that share one piece of its scratch in inference.
+constexpr int kPlanarFrom = 1 << 15;
+constexpr int kPlanarPiece = 1 << 20;
+
+bool mlp32_forward_supported(const MlpShape& s);
+void mlp32_forward(const MlpShape& s, const FwdInput& in, const __half* const* W, const float* const* B,
+                   __half* const* acts, float* out, int N, int out_act, hipStream_t stream, const uint32_t* d_n);
+
+}  // namespace graft

@@ -329,6 +329,18 @@ void TinyMLP::forward(const half* d_unpadded_inputs, float* d_outputs, int batch
     if (batchSize > m_maxBatchSize) throw std::runtime_error("Batch size exceeds maxBatchSize");
     if (batchSize <= 0) return;
     graft::FwdInput in;
+    const MlpShape sh = shape_of(hw_opt);
+    if (graft::mlp_forward_wide(sh)) {
+        // pads the input, saves it as activation 0 and writes the caller's outputs itself
+        in.x = d_unpadded_inputs;
+        in.x_dim = user_opt.inputDim;
+        in.save_x0 = true;
+        in.user = d_outputs;
+        in.user_dim = user_opt.outputDim;
+        graft::mlp_forward(sh, in, d_fwd_weights, d_master_biases, d_activations, d_padded_outputs_float, batchSize,
+                           hw_opt.outputActivation, stream);
+        return;
+    }
     if (user_opt.inputDim != hw_opt.inputDim) {
         graft::pad_f16(d_unpadded_inputs, d_padded_inputs, batchSize, user_opt.inputDim, hw_opt.inputDim, stream);
         in.x = d_padded_inputs;
@@ -337,7 +349,7 @@ void TinyMLP::forward(const half* d_unpadded_inputs, float* d_outputs, int batch
         in.x = d_unpadded_inputs;
         in.save_x0 = true;
     }
-    graft::mlp_forward(shape_of(hw_opt), in, d_fwd_weights, d_master_biases, d_activations, d_padded_outputs_float,
+    graft::mlp_forward(sh, in, d_fwd_weights, d_master_biases, d_activations, d_padded_outputs_float,
                        batchSize, hw_opt.outputActivation, stream);
     if (d_outputs) {
         if (user_opt.outputDim == hw_opt.outputDim)
@@ -364,6 +376,19 @@ void TinyMLP::inference(const half* d_unpadded_inputs, float* d_outputs, int bat
     if (batchSize <= 0) return;
     graft::FwdInput in;
     in.x = d_unpadded_inputs;
+    if (graft::mlp_forward_wide(shape_of(hw_opt)) &&
+        (user_opt.inputDim != hw_opt.inputDim || user_opt.outputDim != hw_opt.outputDim)) {
+        // padded rows are made and dropped inside the kernel
+        in.x_dim = user_opt.inputDim;
+        const bool padded_out = user_opt.outputDim != hw_opt.outputDim;
+        in.user = padded_out ? d_outputs : nullptr;
+        in.user_dim = user_opt.outputDim;
+        float* out = padded_out ? d_padded_outputs_float : d_outputs;
+        if (out)
+            graft::mlp_forward(shape_of(hw_opt), in, d_fwd_weights, d_master_biases, nullptr, out, batchSize,
+                               hw_opt.outputActivation, stream);
+        return;
+    }
     if (user_opt.inputDim != hw_opt.inputDim) {
         graft::pad_f16(d_unpadded_inputs, d_padded_inputs, batchSize, user_opt.inputDim, hw_opt.inputDim, stream);
         in.x = d_padded_inputs;
@@ -508,6 +533,7 @@ TinyMLP::Buffers TinyMLP::buffers() const
 // ===========================================================================
 
 #define META (*static_cast<graft::GridMeta*>(m_meta))
+#define ENCODE (*static_cast<graft::StreamScratch*>(m_encode))
 
 TinyMLPHashGrid::TinyMLPHashGrid(const MLPGridOptions& options, int maxBatchSize, int inferBatchSize,
                                  unsigned int seed, bool isTraining)
@@ -533,6 +559,7 @@ TinyMLPHashGrid::TinyMLPHashGrid(const MLPGridOptions& options, int maxBatchSize
     mlp_opt.activationType = hw_opt.activationType;
     mlp_opt.outputActivation = OUT_ACT_NONE;
     shape_of(mlp_opt).validate();
+    m_encode = new graft::StreamScratch();
     m_meta = new graft::GridMeta(graft::make_grid_meta(hw_opt.tableSize, hw_opt.numLevels, hw_opt.b, hw_opt.lowestSize));
     m_totalHashElements = hw_opt.numLevels * hw_opt.tableSize * hw_opt.featuresLevel;
 
@@ -571,6 +598,7 @@ TinyMLPHashGrid::~TinyMLPHashGrid()
     TT.fw.destroy();
     delete static_cast<Tables*>(h_ptrs);
     delete static_cast<graft::GridMeta*>(m_meta);
+    delete static_cast<graft::StreamScratch*>(m_encode);
     h_ptrs = nullptr;
 }
 
@@ -679,9 +707,13 @@ void TinyMLPHashGrid::forward(const float* d_unpadded_inputs, float* d_outputs, 
     in.pos_stride = 4;
     in.table = d_fwd_hashtable;
     in.meta = &META;
+    in.scratch = &ENCODE.of(stream);
+    const bool wide = graft::mlp_forward_wide(shape_of(mlp_opt));
+    in.user = d_outputs;  // the wide kernel stores the caller's outputs too
+    in.user_dim = user_opt.outputDim;
     graft::mlp_forward(shape_of(mlp_opt), in, d_fwd_weights, d_master_biases, d_activations, d_padded_outputs_float,
                        batchSize, OUT_ACT_NONE, stream);
-    if (d_outputs) {
+    if (d_outputs && !wide) {
         if (user_opt.outputDim == hw_opt.outputDim)
             GRAFT_HIP_CHECK(hipMemcpyAsync(d_outputs, d_padded_outputs_float,
                                            (size_t)batchSize * hw_opt.outputDim * sizeof(float),
@@ -709,14 +741,18 @@ void TinyMLPHashGrid::inference(const float* d_unpadded_inputs, float* d_outputs
     in.pos_stride = user_opt.vectorDim;
     in.table = d_fwd_hashtable;
     in.meta = &META;
+    in.scratch = &ENCODE.of(stream);
     if (user_opt.outputDim == hw_opt.outputDim) {
         if (d_outputs)
             graft::mlp_forward(shape_of(mlp_opt), in, d_fwd_weights, d_master_biases, nullptr, d_outputs, batchSize,
                                OUT_ACT_NONE, stream);
     } else {
+        const bool wide = graft::mlp_forward_wide(shape_of(mlp_opt));
+        in.user = d_outputs;  // the wide kernel stores the caller's outputs too
+        in.user_dim = user_opt.outputDim;
         graft::mlp_forward(shape_of(mlp_opt), in, d_fwd_weights, d_master_biases, nullptr, d_padded_outputs_float,
                            batchSize, OUT_ACT_NONE, stream);
-        if (d_outputs)
+        if (d_outputs && !wide)
             graft::unpad_f32(d_padded_outputs_float, d_outputs, batchSize, hw_opt.outputDim, user_opt.outputDim,
                              stream);
     }

@@ -151,6 +151,7 @@ private:
     void* h_ptrs = nullptr;
     void* m_meta = nullptr;   // hash-grid level table (opaque)
     void* m_scatter = nullptr; // binned-scatter scratch of this instance (opaque)
+    void* m_encode = nullptr;     // per stream: level-major encodings of large batches (opaque)
     void* m_workspace = nullptr;  // partial-sum workspace of the loss and backward (opaque)
 
     void allocate_memory();
