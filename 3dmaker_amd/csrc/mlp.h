@@ -53,7 +53,7 @@ void mlp_backward(const MlpShape& s, const __half* dy, const __half* const* acts
                   hipStream_t stream, const uint32_t* d_n = nullptr, bool accumulate = true,
                   Workspace* ws = nullptr);
 
-// dx = dL/dx alone, bitwise the dx of mlp_backward, for the NeRF head shapes
+// dx = dL/dx alone, with the rounding points of mlp_backward, for the NeRF head shapes
 // (32-64-16, 2 layers; 32-64-8, 3 layers); returns false for other shapes.
 // mlp_backward(..., dx = nullptr) then yields the weight gradients.
 bool mlp_backward_dx(const MlpShape& s, const __half* dy, const __half* const* acts, const __half* const* W,
@@ -67,7 +67,7 @@ void mlp_grad_reduce(const MlpShape& s, const float* ws, int nparts, float* cons
                      bool accumulate, hipStream_t stream);
 
 // The forward of a NeRF step (hash encode + density head, SH gather, colour
-// head) in one launch; bitwise equal to mlp_forward(density), sh_gather,
+// head) in one launch: mlp_forward(density), sh_gather,
 // mlp_forward(colour).  dacts / density_out / cacts / color_in may be null
 // (inference); sigma and color_out are always written.
 struct NerfFwdArgs {
@@ -110,7 +110,7 @@ void nerf_forward(const NerfFwdArgs& a, int N, hipStream_t stream, const uint32_
 
 // The dX part of a NeRF step's backward in one launch: colour dL/dinput,
 // density dL/dy (colour dL/dinput[0..15] + d sigma on the logit, clamped) and
-// dL/d(encoding); bitwise equal to mlp_backward_dx(colour), density_grad,
+// dL/d(encoding): mlp_backward_dx(colour), density_grad,
 // mlp_backward_dx(density).  Only for the head shapes 32-64-64-8 and
 // 32-64-16; returns false for others.
 struct NerfBwdDxArgs {

@@ -20,6 +20,7 @@
 #include "hashgrid.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace graft {
 
@@ -40,12 +41,12 @@ __host__ __device__ __forceinline__ int up32(int d) { return (d + 31) & ~31; }
 
 // The weights in LDS: layer 0's HID rows of up32(in) halves, then the rows of
 // all other layers, HID halves each, one after another (the last layer's
-// padded to a multiple of 16); every row is followed by 8 halves of padding
+// padded to last_rows); every row is followed by 8 halves of padding
 // against bank conflicts.
 __host__ __device__ __forceinline__ int rows0_halves(int hid, int in) { return hid * (up32(in) + 8); }
-__host__ __device__ __forceinline__ int rows_halves(int hid, int in, int out, int layers)
+__host__ __device__ __forceinline__ int rows_halves(int hid, int in, int layers, int last_rows)
 {
-    return rows0_halves(hid, in) + ((layers - 2) * hid + up16(out)) * (hid + 8);
+    return rows0_halves(hid, in) + ((layers - 2) * hid + last_rows) * (hid + 8);
 }
 // First LDS half of layer l's rows, and their pitch.
 template <int HID>
@@ -60,7 +61,8 @@ __device__ __forceinline__ int row_base(int l, int in)
 // they came one after another, and 1,003 samples through 8-128-128-128-8 took
 // 18.4 us instead of 11.4.  All threads call; ends with a barrier.
 template <int HID>
-__device__ __forceinline__ void stage_rows(_Float16* sw, const _Float16* const* W, int in, int out, int layers)
+__device__ __forceinline__ void stage_rows(_Float16* sw, const _Float16* const* W, int in, int out, int layers,
+                                           int last_rows)
 {
     constexpr int kBatch = 12;
     constexpr int C = HID / 8;  // chunks of a row behind layer 0
@@ -72,7 +74,7 @@ __device__ __forceinline__ void stage_rows(_Float16* sw, const _Float16* const* 
     for (int l = 0; l < layers; l++) low |= reinterpret_cast<uintptr_t>(sW[l]);
     const bool vec = __builtin_amdgcn_readfirstlane((int)(low & 15u)) == 0;
     const int C0 = up32(in) >> 3, total0 = HID * C0;
-    const int total = total0 + ((layers - 2) * HID + up16(out)) * C;
+    const int total = total0 + ((layers - 2) * HID + last_rows) * C;
     for (int base = 0; base < total; base += kBatch * (int)blockDim.x) {
         h8 v[kBatch];
         int dst[kBatch];
@@ -170,7 +172,7 @@ __global__ __launch_bounds__(256) void mlp32_fwd_kernel(const Fwd32Params p)
         return ok ? v : 0.f;
     };
     const float b0 = bias(tid), b1 = bias(tid + 256);
-    stage_rows<HID>(sw, p.W, p.in, p.out_dim, p.layers);
+    stage_rows<HID>(sw, p.W, p.in, p.out_dim, p.layers, up16(p.out_dim));
     if (tid < nb) sb[tid] = b0;
     if (tid + 256 < nb) sb[tid + 256] = b1;
     for (int e = tid + 512; e < nb; e += 256) sb[e] = bias(e);
@@ -386,9 +388,299 @@ void pick_fwd32(const Fwd32Params& p, int mode, bool save, int act, int lds, int
     }
 }
 
-int fwd32_bias_base(const MlpShape& s) { return (rows_halves(s.hid, s.in, s.out, s.layers) * 2 + 15) & ~15; }
+int fwd32_bias_base(const MlpShape& s) { return (rows_halves(s.hid, s.in, s.layers, up16(s.out)) * 2 + 15) & ~15; }
 int fwd32_lds(const MlpShape& s) { return fwd32_bias_base(s) + 4 * ((s.layers - 1) * s.hid + up16(s.out)); }
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
+
+// ---------------------------------------------------------------------------
+// backward
+// ---------------------------------------------------------------------------
+
+constexpr int kBwdRows = 128;  // samples of a block's chunk: 32 per wave
+
+struct Bwd32Params {
+    const _Float16* dy;          // [N x out]
+    const _Float16* const* acts; // device array: acts[0] = layer-0 input, acts[l] = H_l
+    const _Float16* const* W;
+    float* ws;                   // [gridDim.x][P] partial dW (all layers) then db
+    _Float16* dx;                // nullable [N x in]
+    const uint32_t* d_n;
+    int N, in, out_dim, layers;
+    int wofs[kMaxLayers], bofs[kMaxLayers];
+    int P, pitch;                // pitch: halves of a row of the exchange buffers
+    int g_base, x_base;          // their byte offsets in LDS
+    int vec_dy;
+};
+
+// Transposing LDS read (16-bit): of the 4 x 16 halves that the 16 lanes of a
+// group name (lane k: row k / 4, columns 4 (k % 4) ..), lane i gets column i.
+typedef short s4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ h4 lds_tr(const _Float16* p)
+{
+    typedef __attribute__((address_space(3))) s4 lds_s4;
+    return __builtin_bit_cast(h4, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4*)p));
+}
+// Eight rows from p (this lane's row and column of lds_tr's 4 x 16) on: the
+// lane's column of rows 0..7.
+__device__ __forceinline__ h8 lds_tr8(const _Float16* p, int pitch)
+{
+    const h4 a = lds_tr(p), b = lds_tr(p + 4 * pitch);
+    return h8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+}
+
+// A block takes 128 samples through all layers.  Per layer every wave puts the
+// dL/dy and the input activations of its 32 samples into LDS as they lie (16
+// bytes per lane); dW = dY^T X then takes its operands, samples along K, with
+// the transposing LDS read, each wave owning a quarter of the layer's 16x16
+// blocks over all 128 samples, and dX = dY W of the wave's own samples takes
+// W^T from the weights' rows the same way.  db is one more column of ones.
+// dW/db stay in registers until the block's last chunk; the next layer's (or
+// chunk's) activations are loaded during the products.
+// What is left is the bytes of dL/dy and activations (33 us for 2^18 samples
+// of 64-64-64-64-64 at a large copy's rate) and two barriers per layer: 76 us,
+// 150 with 2-byte transposing LDS writes and 16x16x16 products before; 65,537
+// samples of 32-64-64-8 21 us, 37 before; 2^18 of 32-64-16 32 us, 33 before.
+template <int HB, int LAYERS>
+__global__ __launch_bounds__(256, HB == 1 ? 4 : HB == 2 ? 2 : 1) void mlp32_bwd_kernel(const Bwd32Params p)
+{
+    constexpr int HID = 32 * HB;
+    constexpr int WO_H = HB == 1 ? 2 : 4, WI_H = 4 / WO_H;  // a hidden layer's waves along o and i
+    constexpr int AH = 2 * HB / WO_H, BH = 2 * HB / WI_H;   // and the blocks of each
+    constexpr int QW = AH * BH;
+    extern __shared__ __align__(16) unsigned char smem[];
+    _Float16* sw = reinterpret_cast<_Float16*>(smem);
+    _Float16* sg = reinterpret_cast<_Float16*>(smem + p.g_base);
+    _Float16* sx = reinterpret_cast<_Float16*>(smem + p.x_base);
+    stage_rows<HID>(sw, p.W, p.in, p.out_dim, LAYERS, up32(p.out_dim));
+
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    const int N = p.d_n ? min((int)*p.d_n, p.N) : p.N;
+    const int nchunks = (N + kBwdRows - 1) / kBwdRows;
+    const int pitch = p.pitch;
+    h8 ones;
+#pragma unroll
+    for (int j = 0; j < 8; j++) ones[j] = (_Float16)1.f;
+    f4 dw[LAYERS][QW], db[LAYERS][AH];
+#pragma unroll
+    for (int l = 0; l < LAYERS; l++) {
+#pragma unroll
+        for (int k = 0; k < QW; k++) dw[l][k] = f4zero();
+#pragma unroll
+        for (int k = 0; k < AH; k++) db[l][k] = f4zero();
+    }
+
+    auto load = [&](const _Float16* src, int width, bool vec, int chunk, h8 (&V)[2][HB]) {
+#pragma unroll
+        for (int t = 0; t < 2; t++) {
+            const int n = chunk * kBwdRows + (wave * 2 + t) * 16 + r;
+#pragma unroll
+            for (int b = 0; b < HB; b++) {
+                V[t][b] = h8zero();
+                const int col = 32 * b + 8 * g;
+                if (n >= N || col >= width) continue;
+                const _Float16* q = src + (size_t)n * width + col;
+                if (vec) {
+                    V[t][b] = *reinterpret_cast<const h8*>(q);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 8; j++)
+                        if (col + j < width) V[t][b][j] = q[j];
+                }
+            }
+        }
+    };
+    auto load_act = [&](int l, int chunk, h8 (&V)[2][HB]) {
+        const _Float16* src = p.acts[l];
+        load(src, l == 0 ? p.in : HID, (reinterpret_cast<uintptr_t>(src) & 15u) == 0, chunk, V);
+    };
+
+    h8 G[2][HB], X[2][HB];
+    int chunk = blockIdx.x;
+    if (chunk < nchunks) {
+        load(p.dy, p.out_dim, p.vec_dy, chunk, G);
+        load_act(LAYERS - 1, chunk, X);
+    }
+    for (; chunk < nchunks; chunk += gridDim.x) {
+        const int next = chunk + gridDim.x;
+        auto layer = [&](auto lc, f4 (&dwl)[QW], f4 (&dbl)[AH]) {
+            constexpr int l = decltype(lc)::value;
+            constexpr bool last = l == LAYERS - 1;
+            const int KO = last ? (p.out_dim + 31) >> 5 : HB;  // 32-blocks of dL/dy
+            const int KI = l == 0 ? (p.in + 31) >> 5 : HB;     // and of the input
+            h8 Xn[2][HB], Gn[2][HB];
+            if constexpr (l > 0) {
+                load_act(l - 1, chunk, Xn);
+            } else if (next < nchunks) {
+                load_act(LAYERS - 1, next, Xn);
+                load(p.dy, p.out_dim, p.vec_dy, next, Gn);
+            }
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const int row = ((wave * 2 + t) * 16 + r) * pitch + 8 * g;
+#pragma unroll
+                for (int b = 0; b < HB; b++) {
+                    if (b < KO) *reinterpret_cast<h8*>(sg + row + 32 * b) = G[t][b];
+                    if (b < KI) *reinterpret_cast<h8*>(sx + row + 32 * b) = X[t][b];
+                }
+            }
+            __syncthreads();
+
+            // dW, db: this wave's blocks (wo + WO a, wi + WI b) over the chunk's samples
+            const int OB = last ? up16(p.out_dim) >> 4 : 2 * HB, IB = l == 0 ? up16(p.in) >> 4 : 2 * HB;
+            const int WO = last ? min(OB, 4) : WO_H, WI = 4 / WO;
+            const int wo = wave & (WO - 1), wi = wave / WO;
+            const int NB = (IB + WI - 1) / WI;  // blocks of the wave along i
+            const _Float16* tg = sg + (8 * g + (r >> 2)) * pitch + 4 * (r & 3);
+            const _Float16* tx = sx + (8 * g + (r >> 2)) * pitch + 4 * (r & 3);
+#pragma unroll 1
+            for (int ks = 0; ks < kBwdRows / 32; ks++) {
+                const int at = 32 * ks * pitch;
+                if constexpr (!last) {
+#pragma unroll
+                    for (int a = 0; a < AH; a++) {
+                        const h8 A = lds_tr8(tg + at + 16 * (wo + WO_H * a), pitch);
+                        if (wi == 0) dbl[a] = mfma32(A, ones, dbl[a]);
+#pragma unroll
+                        for (int b = 0; b < BH; b++)
+                            if (wi + WI_H * b < IB)
+                                dwl[a * BH + b] = mfma32(A, lds_tr8(tx + at + 16 * (wi + WI_H * b), pitch), dwl[a * BH + b]);
+                    }
+                } else {
+#pragma unroll
+                    for (int k = 0; k < QW; k++) {
+                        const int a = k / NB, b = k - a * NB;
+                        if (wo + WO * a >= OB || wi + WI * b >= IB) continue;
+                        const h8 A = lds_tr8(tg + at + 16 * (wo + WO * a), pitch);
+                        dwl[k] = mfma32(A, lds_tr8(tx + at + 16 * (wi + WI * b), pitch), dwl[k]);
+                    }
+#pragma unroll
+                    for (int a = 0; a < AH; a++)
+                        if (wi == 0 && wo + WO * a < OB)
+                            dbl[a] = mfma32(lds_tr8(tg + at + 16 * (wo + WO * a), pitch), ones, dbl[a]);
+                }
+            }
+            // dX of this wave's 32 samples, rounded to fp16, masked by the input
+            if (l > 0 || p.dx != nullptr) {
+                const int wp = l == 0 ? 32 * KI + 8 : HID + 8;
+                const _Float16* w = sw + row_base<HID>(l, p.in) + (8 * g + (r >> 2)) * wp + 8 * (r & 3);
+                h8 D[2][HB];
+#pragma unroll
+                for (int q = 0; q < HB; q++) {
+                    if (q >= KI) continue;
+                    f4 acc[2][2];
+#pragma unroll
+                    for (int t = 0; t < 2; t++)
+#pragma unroll
+                        for (int m = 0; m < 2; m++) acc[t][m] = f4zero();
+#pragma unroll
+                    for (int kb = 0; kb < HB; kb++) {
+                        if (kb >= KO) continue;
+#pragma unroll
+                        for (int m = 0; m < 2; m++) {
+                            const h8 A = lds_tr8(w + 32 * kb * wp + 32 * q + 4 * m, wp);
+#pragma unroll
+                            for (int t = 0; t < 2; t++) acc[t][m] = mfma32(A, G[t][kb], acc[t][m]);
+                        }
+                    }
+#pragma unroll
+                    for (int t = 0; t < 2; t++)
+#pragma unroll
+                        for (int j = 0; j < 8; j++) {
+                            const _Float16 v = to_h(acc[t][j >> 2][j & 3]);
+                            D[t][q][j] = l > 0 && !(X[t][q][j] > (_Float16)0.f) ? (_Float16)0.f : v;
+                        }
+                }
+                if (l == 0) {
+#pragma unroll
+                    for (int t = 0; t < 2; t++) {
+                        const int n = chunk * kBwdRows + (wave * 2 + t) * 16 + r;
+#pragma unroll
+                        for (int q = 0; q < HB; q++) {
+                            const int col = 32 * q + 8 * g;
+                            if (q < KI && n < N && col < p.in) st_row8(p.dx + (size_t)n * p.in + col, D[t][q]);
+                        }
+                    }
+                } else {
+#pragma unroll
+                    for (int t = 0; t < 2; t++)
+#pragma unroll
+                        for (int q = 0; q < HB; q++) Gn[t][q] = D[t][q];
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int b = 0; b < HB; b++) {
+                    G[t][b] = Gn[t][b];
+                    X[t][b] = Xn[t][b];
+                }
+        };
+        if constexpr (LAYERS > 3) layer(std::integral_constant<int, 3>{}, dw[3], db[3]);
+        if constexpr (LAYERS > 2) layer(std::integral_constant<int, 2>{}, dw[2], db[2]);
+        layer(std::integral_constant<int, 1>{}, dw[1], db[1]);
+        layer(std::integral_constant<int, 0>{}, dw[0], db[0]);
+    }
+
+    float* dst = p.ws + (size_t)blockIdx.x * p.P;
+#pragma unroll
+    for (int l = 0; l < LAYERS; l++) {
+        const bool last = l == LAYERS - 1;
+        const int in_l = l == 0 ? p.in : HID, out_l = last ? p.out_dim : HID;
+        const int OB = last ? up16(p.out_dim) >> 4 : 2 * HB, IB = l == 0 ? up16(p.in) >> 4 : 2 * HB;
+        const int WO = last ? min(OB, 4) : WO_H, WI = 4 / WO;
+        const int wo = wave & (WO - 1), wi = wave / WO;
+        const int NB = last ? (IB + WI - 1) / WI : BH;
+#pragma unroll
+        for (int k = 0; k < QW; k++) {
+            const int a = k / NB, b = k - a * NB;
+            const int i = 16 * (wi + WI * b) + r;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int o = 16 * (wo + WO * a) + 4 * g + j;
+                if (o < out_l && i < in_l) dst[p.wofs[l] + o * in_l + i] = dw[l][k][j];
+            }
+        }
+#pragma unroll
+        for (int a = 0; a < AH; a++) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int o = 16 * (wo + WO * a) + 4 * g + j;
+                if (wi == 0 && r == 0 && o < out_l) dst[p.bofs[l] + o] = db[l][a][j];
+            }
+        }
+    }
+}
+
+// LDS of the backward: weights with the last layer's rows padded for the
+// 32-wide products, then the two exchange buffers.
+struct Bwd32Lds {
+    int pitch, g_base, x_base, bytes;
+};
+
+Bwd32Lds bwd32_lds(const MlpShape& s)
+{
+    Bwd32Lds o{};
+    o.pitch = s.hid + 8;
+    o.g_base = (rows_halves(s.hid, s.in, s.layers, up32(s.out)) * 2 + 15) & ~15;
+    o.x_base = o.g_base + kBwdRows * o.pitch * 2;
+    o.bytes = o.x_base + kBwdRows * o.pitch * 2;
+    return o;
+}
+
+template <int HB>
+void launch_bwd32(const Bwd32Params& p, int lds, int blocks, hipStream_t stream)
+{
+    if (p.layers == 2) {
+        hipLaunchKernelGGL((mlp32_bwd_kernel<HB, 2>), dim3(blocks), dim3(256), lds, stream, p);
+    } else if constexpr (HB < 4) {
+        if (p.layers == 3)
+            hipLaunchKernelGGL((mlp32_bwd_kernel<HB, 3>), dim3(blocks), dim3(256), lds, stream, p);
+        else
+            hipLaunchKernelGGL((mlp32_bwd_kernel<HB, 4>), dim3(blocks), dim3(256), lds, stream, p);
+    }
+    GRAFT_LAUNCH_CHECK();
+}
 
 }  // namespace
 
@@ -469,6 +761,53 @@ void mlp32_forward(const MlpShape& s, const FwdInput& in, const __half* const* W
     }
     p.pos = in.pos;
     run(kFused, 0, N);
+}
+
+// Widths up to the hidden one (32 at least) at both ends, and layers whose
+// dW fits the registers: four of width 64, two of 128.  What lies outside is
+// mlp.hip's.
+bool mlp32_backward_supported(const MlpShape& s)
+{
+    if (s.hid != 32 && s.hid != 64 && s.hid != 128) return false;
+    if (s.layers < 2 || s.layers > (s.hid == 128 ? 2 : 4)) return false;
+    if (s.in % 8 || up32(s.in) > s.hid || s.out % 4 || up32(s.out) > s.hid) return false;
+    const int ob = up16(s.out) / 16;
+    if (ob & (ob - 1)) return false;
+    return bwd32_lds(s).bytes + kStaticLds <= max_lds_per_block();
+}
+
+int mlp32_backward(const MlpShape& s, const Mlp32Backward& a, int N, hipStream_t stream)
+{
+    const Bwd32Lds lds = bwd32_lds(s);
+    const int nchunks = (N + kBwdRows - 1) / kBwdRows;
+    const int per_cu = std::max(1, std::min(s.hid == 32 ? 4 : 2, max_lds_per_block() / (lds.bytes + kStaticLds)));
+    const int blocks = std::max(1, std::min(nchunks, num_cus() * per_cu));
+    Bwd32Params p{};
+    p.dy = reinterpret_cast<const _Float16*>(a.dy);
+    p.acts = reinterpret_cast<const _Float16* const*>(a.acts);
+    p.W = reinterpret_cast<const _Float16* const*>(a.W);
+    p.dx = reinterpret_cast<_Float16*>(a.dx);
+    p.d_n = a.d_n;
+    p.N = N;
+    p.in = s.in;
+    p.out_dim = s.out;
+    p.layers = s.layers;
+    for (int l = 0; l < s.layers; l++) {
+        p.wofs[l] = a.wofs[l];
+        p.bofs[l] = a.bofs[l];
+    }
+    p.P = a.P;
+    p.pitch = lds.pitch;
+    p.g_base = lds.g_base;
+    p.x_base = lds.x_base;
+    p.vec_dy = s.out % 8 == 0 && aligned16(a.dy);
+    p.ws = static_cast<float*>(a.ws->get((size_t)blocks * a.P * sizeof(float)));
+    switch (s.hid) {
+        case 32: launch_bwd32<1>(p, lds.bytes, blocks, stream); break;
+        case 64: launch_bwd32<2>(p, lds.bytes, blocks, stream); break;
+        default: launch_bwd32<4>(p, lds.bytes, blocks, stream); break;
+    }
+    return blocks;
 }
 
 }  // namespace graft
