@@ -556,7 +556,8 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
     // since the last call) for the first step's forward
     auto pack_heads = [&](hipStream_t s) {
         graft::nerf_heads_pack(
-            graft::NerfHeadsWeights{db.fwd_weights, db.master_biases, cb.fwd_weights, cb.master_biases},
+            graft::NerfHeadsWeights{db.fwd_weights, db.master_biases, cb.fwd_weights, cb.master_biases, cshape.hid,
+                                    cshape.layers},
             b.heads_packed, s);
     };
     if (b.heads_packed) pack_heads(stream);
@@ -703,6 +704,8 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
         bx.denc = db.dx_out;
         graft::NerfHeadsBwd hb;
         hb.packed = b.heads_packed;
+        hb.color_hidden = cshape.hid;
+        hb.color_layers = cshape.layers;
         hb.enc = b.enc_planar;
         hb.enc_plane = (int)Bn;
         hb.levels = b.meta.numLevels;

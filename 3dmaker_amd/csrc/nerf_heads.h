@@ -1,4 +1,5 @@
-// The NeRF training step's two heads (density 32-64-16, colour 32-64-64-8) on
+// The NeRF training step's two heads (density 32-64-16, colour 32-H-8 or
+// 32-H-H-8 with H = 32 or 64) on
 // the 16x16x32 fp16 MFMA (nerf_heads.hip).  The forward stores only sigma,
 // the density output, the colour output and the colour input; both backward
 // kernels recompute a tile's hidden activations from the encodings and the
@@ -16,10 +17,12 @@ struct NerfHeadsWeights {
     const float* const* dB;
     const __half* const* cW;
     const float* const* cB;
+    int color_hidden = 64, color_layers = 3;
 };
 
 struct NerfHeadsFwd {
     const void* packed;            // nerf_heads_pack output
+    int color_hidden = 64, color_layers = 3;
     const __half* enc;             // [levels][enc_plane] feature pairs (hash_encode_planar)
     int enc_plane = 0;
     int levels = 16;
@@ -37,6 +40,7 @@ struct NerfHeadsFwd {
 
 struct NerfHeadsBwd {
     const void* packed;
+    int color_hidden = 64, color_layers = 3;
     const __half* enc;
     int enc_plane = 0;
     int levels = 16;

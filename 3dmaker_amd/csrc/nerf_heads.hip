@@ -1,6 +1,7 @@
 // The two NeRF heads of the training step on gfx950's 16x16x32 fp16 MFMA:
-// density 32-64-16 (ReLU) and colour 32-64-64-8 (ReLU, sigmoid output), the
-// shapes of InstantNerf (networkFusionHashtable.cu:441-682,
+// density 32-64-16 (ReLU) and colour 32-H(-H)-8 (ReLU, sigmoid output), H = 64
+// or 32, two or three layers: the shapes of InstantNerf's defaults (64, two),
+// of INerfTrainer (32, three) and of wider models (networkFusionHashtable.cu:441-682,
 // networkFusion.cu:197-355, networkFusionBackward.cu:49-646,
 // networkFusionBackwardHashtable.cu:71-781).
 //
@@ -40,37 +41,64 @@ namespace {
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 
 constexpr int DIN = 32, DHID = 64, DOUT = 16;  // density head
-constexpr int CIN = 32, CHID = 64, COUT = 8;   // colour head (hardware output width)
+constexpr int CIN = 32, COUT = 8;              // colour head (hardware output width)
 
-// forward fragments (A = W, rows = outputs, slots = inputs)
-constexpr int FD0 = 0;   // density L0: mt 0..3
-constexpr int FD1 = 4;   // density L1: kb 0..1
-constexpr int FC0 = 6;   // colour L0: mt 0..3
-constexpr int FC1 = 10;  // colour L1: 2 mt + kb
-constexpr int FC2 = 18;  // colour L2: kb 0..1
-constexpr int kFwdFrags = 20;
-// transposed fragments (A = W^T, rows = inputs, slots = outputs)
-constexpr int TC2 = 0;   // colour L2^T: mt 0..3 (inputs 0..63), outputs 0..7
-constexpr int TC1 = 4;   // colour L1^T: 2 mt + kb
-constexpr int TC0 = 12;  // colour L0^T, logit inputs 0..15 only: kb 0..1
-constexpr int TD1 = 14;  // density L1^T: mt 0..3, outputs 0..15
-constexpr int TD0 = 18;  // density L0^T: 2 mt + kb (mt 0..1)
-constexpr int kTrFrags = 22;
+// density forward fragments (A = W, rows = outputs, slots = inputs)
+constexpr int FD0 = 0;   // L0: mt 0..3
+constexpr int FD1 = 4;   // L1: kb 0..1
 // bias blocks (rows 16 mt + 4 g + j in lane group g)
-constexpr int BD0 = 0, BD1 = 4, BC0 = 5, BC1 = 9, BC2 = 13;
-constexpr int kBiasBlocks = 14;
+constexpr int BD0 = 0, BD1 = 4;
+constexpr int kDensityBiasBlocks = 5;
 
-constexpr size_t kFwdBytes = (size_t)kFwdFrags * 64 * 16;
-constexpr size_t kTrBytes = (size_t)kTrFrags * 64 * 16;
-constexpr size_t kBiasBytes = (size_t)kBiasBlocks * 4 * 16;
+// A colour head 32 - CH (- CH) - 8 of CL layers: where its fragments, bias
+// blocks and parameters lie.  L0 is the first layer, L2 the last, L1 the one
+// between (CL == 3 only).
+template <int CH, int CL>
+struct ColorHead {
+    static constexpr int CHID = CH, LAYERS = CL, H16 = CH / 16, KB = CH / 32;
+    static constexpr bool MID = CL == 3;
+    // forward fragments
+    static constexpr int FC0 = 6;                              // L0: mt
+    static constexpr int FC1 = FC0 + H16;                      // L1: KB mt + kb
+    static constexpr int FC2 = FC1 + (MID ? H16 * KB : 0);     // L2: kb
+    static constexpr int kFwdFrags = FC2 + KB;
+    // transposed fragments (A = W^T, rows = inputs, slots = outputs)
+    static constexpr int TC2 = 0;                              // L2^T: mt (inputs), outputs 0..7
+    static constexpr int TC1 = TC2 + H16;                      // L1^T: KB mt + kb
+    static constexpr int TC0 = TC1 + (MID ? H16 * KB : 0);     // L0^T, logit inputs 0..15 only: kb
+    static constexpr int TD1 = TC0 + KB;                       // density L1^T: mt 0..3, outputs 0..15
+    static constexpr int TD0 = TD1 + 4;                        // density L0^T: 2 mt + kb (mt 0..1)
+    static constexpr int kTrFrags = TD0 + 4;
+    // bias blocks
+    static constexpr int BC0 = kDensityBiasBlocks, BC1 = BC0 + H16, BC2 = BC1 + (MID ? H16 : 0);
+    static constexpr int kBiasBlocks = BC2 + 1;
+    // parameters in mlp_grad_reduce's order: W of every layer (row-major
+    // [out][in]), then b of every layer
+    static constexpr int PC_W0 = 0, PC_W1 = PC_W0 + CH * CIN, PC_W2 = PC_W1 + (MID ? CH * CH : 0);
+    static constexpr int PC_B0 = PC_W2 + COUT * CH, PC_B1 = PC_B0 + CH, PC_B2 = PC_B1 + (MID ? CH : 0);
+    static constexpr int PC = PC_B2 + COUT;
+};
 
-// parameters of each head in mlp_grad_reduce's order: W of every layer
-// (row-major [out][in]), then b of every layer
+// The packed buffer has room for the largest head whatever it holds.
+using LargestHead = ColorHead<64, 3>;
+constexpr size_t kFwdBytes = (size_t)LargestHead::kFwdFrags * 64 * 16;
+constexpr size_t kTrBytes = (size_t)LargestHead::kTrFrags * 64 * 16;
+constexpr size_t kBiasBytes = (size_t)LargestHead::kBiasBlocks * 4 * 16;
+
+// f(ColorHead<...>{}) for the colour head of that width and depth
+template <class F>
+void with_head(int hidden, int layers, F&& f)
+{
+    if (hidden == 64 && layers == 3) f(ColorHead<64, 3>{});
+    else if (hidden == 32 && layers == 3) f(ColorHead<32, 3>{});
+    else if (hidden == 64 && layers == 2) f(ColorHead<64, 2>{});
+    else if (hidden == 32 && layers == 2) f(ColorHead<32, 2>{});
+    else throw std::runtime_error("NeRF heads: unsupported colour head");
+}
+
+// density parameters in the same order
 constexpr int PD_W0 = 0, PD_W1 = PD_W0 + DHID * DIN, PD_B0 = PD_W1 + DOUT * DHID, PD_B1 = PD_B0 + DHID;
 constexpr int PD = PD_B1 + DOUT;  // 3152
-constexpr int PC_W0 = 0, PC_W1 = PC_W0 + CHID * CIN, PC_W2 = PC_W1 + CHID * CHID, PC_B0 = PC_W2 + COUT * CHID;
-constexpr int PC_B1 = PC_B0 + CHID, PC_B2 = PC_B1 + CHID;
-constexpr int PC = PC_B2 + COUT;  // 6792
 
 __host__ __device__ constexpr int kslot(int kb, int g, int j) { return 32 * kb + (j < 4 ? 4 * g + j : 12 + 4 * g + j); }
 
@@ -131,9 +159,9 @@ struct PackParams {
     const float* const* dB;
     const _Float16* const* cW;
     const float* const* cB;
-    h8* fwd;   // [kFwdFrags][64]
-    h8* tr;    // [kTrFrags][64]
-    f4* bias;  // [kBiasBlocks][4]
+    h8* fwd;   // [forward fragments][64]
+    h8* tr;    // [transposed fragments][64]
+    f4* bias;  // [bias blocks][4]
     bool density_only;  // the density head's forward fragments and biases only
 };
 
@@ -143,11 +171,14 @@ __device__ __forceinline__ _Float16 wat(const _Float16* W, int out, int in, int 
     return (row < out && col < in) ? W[row * in + col] : (_Float16)0.f;
 }
 
+template <class S>
 __global__ __launch_bounds__(256) void pack_kernel(const PackParams p)
 {
+    constexpr int kFwdFrags = S::kFwdFrags, kTrFrags = S::kTrFrags, kBiasBlocks = S::kBiasBlocks, CHID = S::CHID;
+    constexpr int kLast = S::LAYERS - 1, KB = S::KB;
     const int t = blockIdx.x * 256 + threadIdx.x;
     const int nf = (kFwdFrags + kTrFrags) * 64;
-    if (p.density_only && (t < nf ? (t >> 6) >= FC0 : ((t - nf) >> 2) >= BC0)) return;
+    if (p.density_only && (t < nf ? (t >> 6) >= S::FC0 : ((t - nf) >> 2) >= S::BC0)) return;
     if (t < nf) {
         const int lane = t & 63, f = t >> 6, m = lane & 15, g = lane >> 4;
         h8 v;
@@ -155,10 +186,10 @@ __global__ __launch_bounds__(256) void pack_kernel(const PackParams p)
             const _Float16* W;
             int out, in, mt, kb;
             if (f < FD1) { W = p.dW[0]; out = DHID; in = DIN; mt = f - FD0; kb = 0; }
-            else if (f < FC0) { W = p.dW[1]; out = DOUT; in = DHID; mt = 0; kb = f - FD1; }
-            else if (f < FC1) { W = p.cW[0]; out = CHID; in = CIN; mt = f - FC0; kb = 0; }
-            else if (f < FC2) { W = p.cW[1]; out = CHID; in = CHID; mt = (f - FC1) >> 1; kb = (f - FC1) & 1; }
-            else { W = p.cW[2]; out = COUT; in = CHID; mt = 0; kb = f - FC2; }
+            else if (f < S::FC0) { W = p.dW[1]; out = DOUT; in = DHID; mt = 0; kb = f - FD1; }
+            else if (f < S::FC1) { W = p.cW[0]; out = CHID; in = CIN; mt = f - S::FC0; kb = 0; }
+            else if (f < S::FC2) { W = p.cW[1]; out = CHID; in = CHID; mt = (f - S::FC1) / KB; kb = (f - S::FC1) % KB; }
+            else { W = p.cW[kLast]; out = COUT; in = CHID; mt = 0; kb = f - S::FC2; }
 #pragma unroll
             for (int j = 0; j < 8; j++) v[j] = wat(W, out, in, 16 * mt + m, kslot(kb, g, j));
             p.fwd[f * 64 + lane] = v;
@@ -166,11 +197,11 @@ __global__ __launch_bounds__(256) void pack_kernel(const PackParams p)
             const int q = f - kFwdFrags;
             const _Float16* W;
             int out, in, mt, kb;
-            if (q < TC1) { W = p.cW[2]; out = COUT; in = CHID; mt = q - TC2; kb = 0; }
-            else if (q < TC0) { W = p.cW[1]; out = CHID; in = CHID; mt = (q - TC1) >> 1; kb = (q - TC1) & 1; }
-            else if (q < TD1) { W = p.cW[0]; out = CHID; in = CIN; mt = 0; kb = q - TC0; }
-            else if (q < TD0) { W = p.dW[1]; out = DOUT; in = DHID; mt = q - TD1; kb = 0; }
-            else { W = p.dW[0]; out = DHID; in = DIN; mt = (q - TD0) >> 1; kb = (q - TD0) & 1; }
+            if (q < S::TC1) { W = p.cW[kLast]; out = COUT; in = CHID; mt = q - S::TC2; kb = 0; }
+            else if (q < S::TC0) { W = p.cW[1]; out = CHID; in = CHID; mt = (q - S::TC1) / KB; kb = (q - S::TC1) % KB; }
+            else if (q < S::TD1) { W = p.cW[0]; out = CHID; in = CIN; mt = 0; kb = q - S::TC0; }
+            else if (q < S::TD0) { W = p.dW[1]; out = DOUT; in = DHID; mt = q - S::TD1; kb = 0; }
+            else { W = p.dW[0]; out = DHID; in = DIN; mt = (q - S::TD0) >> 1; kb = (q - S::TD0) & 1; }
             // rows = inputs, slots = outputs
 #pragma unroll
             for (int j = 0; j < 8; j++) v[j] = wat(W, out, in, kslot(kb, g, j), 16 * mt + m);
@@ -184,10 +215,10 @@ __global__ __launch_bounds__(256) void pack_kernel(const PackParams p)
         const float* B;
         int out, mt;
         if (b < BD1) { B = p.dB[0]; out = DHID; mt = b - BD0; }
-        else if (b < BC0) { B = p.dB[1]; out = DOUT; mt = 0; }
-        else if (b < BC1) { B = p.cB[0]; out = CHID; mt = b - BC0; }
-        else if (b < BC2) { B = p.cB[1]; out = CHID; mt = b - BC1; }
-        else { B = p.cB[2]; out = COUT; mt = 0; }
+        else if (b < S::BC0) { B = p.dB[1]; out = DOUT; mt = 0; }
+        else if (b < S::BC1) { B = p.cB[0]; out = CHID; mt = b - S::BC0; }
+        else if (b < S::BC2) { B = p.cB[1]; out = CHID; mt = b - S::BC1; }
+        else { B = p.cB[kLast]; out = COUT; mt = 0; }
         f4 v;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -202,8 +233,9 @@ __global__ __launch_bounds__(256) void pack_kernel(const PackParams p)
 // one tile through both heads
 // ---------------------------------------------------------------------------
 
+template <class S>
 struct Weights {
-    h8 F[kFwdFrags];
+    h8 F[S::kFwdFrags];
 };
 
 // The forward fragments staged in LDS, read where they are used.
@@ -216,13 +248,14 @@ struct LdsWeights {
 };
 
 // The forward values of one tile the backward needs.
+template <class S>
 struct Acts {
     h8 enc;      // density input (kslot order)
     h8 hd[2];    // density hidden
     f4 y;        // density output block (pre-sanitise logits, fp32, + bias)
     h8 cin;      // colour input: sanitised logits | SH
-    h8 h1[2];    // colour hidden 1
-    h8 h2[2];    // colour hidden 2
+    h8 h1[S::KB];  // first colour hidden layer
+    h8 h2[S::KB];  // last colour hidden layer (the same one when there are two layers)
     f4 rgb[1];   // colour output rows 4 g .. 4 g + 3 (pre-activation), lanes g < 2
 };
 
@@ -271,8 +304,35 @@ __device__ __forceinline__ h4 sh_quad(float x, float y, float z, int g)
     return s;
 }
 
-__device__ __forceinline__ void forward_tile(const Weights& w, const f4* __restrict__ sbias, const TileIn& in,
-                                             int g, Acts& a)
+// The colour head's hidden layers from its input.
+// FW: the forward fragments, w.F[q] -> h8 (registers or LDS)
+template <class S, class FW>
+__device__ __forceinline__ void color_hidden(const FW& w, const f4* __restrict__ sbias, int g, Acts<S>& a)
+{
+    f4 c0[S::H16];
+#pragma unroll
+    for (int mt = 0; mt < S::H16; mt++) c0[mt] = mfma32(w.F[S::FC0 + mt], a.cin, sbias[(S::BC0 + mt) * 4 + g]);
+#pragma unroll
+    for (int kb = 0; kb < S::KB; kb++) a.h1[kb] = cat(relu_h4(c0[2 * kb]), relu_h4(c0[2 * kb + 1]));
+    if constexpr (S::MID) {
+        f4 c1[S::H16];
+#pragma unroll
+        for (int mt = 0; mt < S::H16; mt++) {
+            c1[mt] = sbias[(S::BC1 + mt) * 4 + g];
+#pragma unroll
+            for (int kb = 0; kb < S::KB; kb++) c1[mt] = mfma32(w.F[S::FC1 + S::KB * mt + kb], a.h1[kb], c1[mt]);
+        }
+#pragma unroll
+        for (int kb = 0; kb < S::KB; kb++) a.h2[kb] = cat(relu_h4(c1[2 * kb]), relu_h4(c1[2 * kb + 1]));
+    } else {
+#pragma unroll
+        for (int kb = 0; kb < S::KB; kb++) a.h2[kb] = a.h1[kb];
+    }
+}
+
+template <class S>
+__device__ __forceinline__ void forward_tile(const Weights<S>& w, const f4* __restrict__ sbias, const TileIn& in,
+                                             int g, Acts<S>& a)
 {
     a.enc = in.enc;
     // density L0 (32 -> 64)
@@ -289,34 +349,20 @@ __device__ __forceinline__ void forward_tile(const Weights& w, const f4* __restr
 #pragma unroll
     for (int j = 0; j < 4; j++) lg[j] = to_h(sanitize_logit(y[j]));
     a.cin = cat(lg, sh_quad(in.dx, in.dy, in.dz, g));
-    // colour L0 (32 -> 64)
-    f4 c0[4];
+    color_hidden<S>(w, sbias, g, a);
+    // last colour layer (-> 8)
+    f4 o = sbias[S::BC2 * 4 + g];
 #pragma unroll
-    for (int mt = 0; mt < 4; mt++) c0[mt] = mfma32(w.F[FC0 + mt], a.cin, sbias[(BC0 + mt) * 4 + g]);
-    a.h1[0] = cat(relu_h4(c0[0]), relu_h4(c0[1]));
-    a.h1[1] = cat(relu_h4(c0[2]), relu_h4(c0[3]));
-    // colour L1 (64 -> 64)
-    f4 c1[4];
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++) {
-        c1[mt] = mfma32(w.F[FC1 + 2 * mt], a.h1[0], sbias[(BC1 + mt) * 4 + g]);
-        c1[mt] = mfma32(w.F[FC1 + 2 * mt + 1], a.h1[1], c1[mt]);
-    }
-    a.h2[0] = cat(relu_h4(c1[0]), relu_h4(c1[1]));
-    a.h2[1] = cat(relu_h4(c1[2]), relu_h4(c1[3]));
-    // colour L2 (64 -> 8)
-    f4 o = mfma32(w.F[FC2 + 0], a.h2[0], sbias[BC2 * 4 + g]);
-    o = mfma32(w.F[FC2 + 1], a.h2[1], o);
+    for (int kb = 0; kb < S::KB; kb++) o = mfma32(w.F[S::FC2 + kb], a.h2[kb], o);
     a.rgb[0] = o;
 }
 
 // The activations the backward needs, from the tile's encodings and the
 // colour input the forward stored: the density hidden layer and both colour
 // hidden layers (the same operations as forward_tile, so the same bits).
-// FW: the forward fragments, w.F[q] -> h8 (registers or LDS)
-template <class FW>
+template <class S, class FW>
 __device__ __forceinline__ void recompute_tile(const FW& w, const f4* __restrict__ sbias, h8 enc, h8 cin, int g,
-                                               Acts& a)
+                                               Acts<S>& a)
 {
     a.enc = enc;
     a.cin = cin;
@@ -325,19 +371,7 @@ __device__ __forceinline__ void recompute_tile(const FW& w, const f4* __restrict
     for (int mt = 0; mt < 4; mt++) d0[mt] = mfma32(w.F[FD0 + mt], enc, sbias[(BD0 + mt) * 4 + g]);
     a.hd[0] = cat(relu_h4(d0[0]), relu_h4(d0[1]));
     a.hd[1] = cat(relu_h4(d0[2]), relu_h4(d0[3]));
-    f4 c0[4];
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++) c0[mt] = mfma32(w.F[FC0 + mt], cin, sbias[(BC0 + mt) * 4 + g]);
-    a.h1[0] = cat(relu_h4(c0[0]), relu_h4(c0[1]));
-    a.h1[1] = cat(relu_h4(c0[2]), relu_h4(c0[3]));
-    f4 c1[4];
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++) {
-        c1[mt] = mfma32(w.F[FC1 + 2 * mt], a.h1[0], sbias[(BC1 + mt) * 4 + g]);
-        c1[mt] = mfma32(w.F[FC1 + 2 * mt + 1], a.h1[1], c1[mt]);
-    }
-    a.h2[0] = cat(relu_h4(c1[0]), relu_h4(c1[1]));
-    a.h2[1] = cat(relu_h4(c1[2]), relu_h4(c1[3]));
+    color_hidden<S>(w, sbias, g, a);
 }
 
 // The inputs of one tile's backward, all indexed by the sample.
@@ -349,41 +383,53 @@ struct BwdIn {
 // The dL/dy blocks of every layer of one tile (fp16, masked as the dX chain
 // passes them on) and dL/d(encoding).
 struct Grads {
-    h8 c2;       // colour L2 output (cdy, slots 0..3 of lane groups 0, 1)
-    h4 c1[4];    // colour L1 output
-    h4 c0[4];    // colour L0 output
     h4 d1;       // density L1 output (dL/dy of the density head)
     h4 d0[4];    // density L0 output
     h4 cx;       // colour dL/d(input) for the logit features 4 g .. 4 g + 3
     h4 denc[2];  // dL/d(encoding), blocks 0..1
 };
 
-// T: the transposed fragments staged in LDS ([kTrFrags][64] h8)
-template <bool FULL_DENC>
-__device__ __forceinline__ void backward_tile(const h8* T, int lane, const Acts& a, h8 cdy, float ds, Grads& gr)
+// The colour dX chain of one tile: dL/dy of the last hidden layer (c1; masked
+// by h2 > 0) and of the first one (c0; masked by h1 > 0), the same blocks when
+// there are two layers.
+// T: the transposed fragments staged in LDS ([S::kTrFrags][64] h8)
+template <class S>
+__device__ __forceinline__ void color_dx(const h8* T, int lane, const Acts<S>& a, h8 cdy, h4 (&c1)[S::H16],
+                                         h4 (&c0)[S::H16])
+{
+    const f4 z = f4zero();
+    auto half = [](const h8* v, int b) { return (b & 1) ? hi4(v[b >> 1]) : lo4(v[b >> 1]); };
+#pragma unroll
+    for (int mt = 0; mt < S::H16; mt++) c1[mt] = mask_h4(mfma32(T[(S::TC2 + mt) * 64 + lane], cdy, z), half(a.h2, mt));
+    if constexpr (S::MID) {
+        h8 g1[S::KB];
+#pragma unroll
+        for (int kb = 0; kb < S::KB; kb++) g1[kb] = cat(c1[2 * kb], c1[2 * kb + 1]);
+#pragma unroll
+        for (int mt = 0; mt < S::H16; mt++) {
+            f4 d = z;
+#pragma unroll
+            for (int kb = 0; kb < S::KB; kb++) d = mfma32(T[(S::TC1 + S::KB * mt + kb) * 64 + lane], g1[kb], d);
+            c0[mt] = mask_h4(d, half(a.h1, mt));
+        }
+    } else {
+#pragma unroll
+        for (int mt = 0; mt < S::H16; mt++) c0[mt] = c1[mt];
+    }
+}
+
+template <class S, bool FULL_DENC>
+__device__ __forceinline__ void backward_tile(const h8* T, int lane, const Acts<S>& a, h8 cdy, float ds, Grads& gr)
 {
     const int g = lane >> 4;
     const f4 z = f4zero();
     auto TF = [&](int q) { return T[q * 64 + lane]; };
-    gr.c2 = cdy;
-    // colour L2^T: dX2 (64) masked by h2 > 0 -> dY1
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++) {
-        const f4 d = mfma32(TF(TC2 + mt), cdy, z);
-        gr.c1[mt] = mask_h4(d, (mt & 1) ? hi4(a.h2[mt >> 1]) : lo4(a.h2[mt >> 1]));
-    }
-    const h8 g1[2] = {cat(gr.c1[0], gr.c1[1]), cat(gr.c1[2], gr.c1[3])};
-    // colour L1^T: dX1 masked by h1 > 0 -> dY0
-#pragma unroll
-    for (int mt = 0; mt < 4; mt++) {
-        f4 d = mfma32(TF(TC1 + 2 * mt), g1[0], z);
-        d = mfma32(TF(TC1 + 2 * mt + 1), g1[1], d);
-        gr.c0[mt] = mask_h4(d, (mt & 1) ? hi4(a.h1[mt >> 1]) : lo4(a.h1[mt >> 1]));
-    }
-    const h8 g0[2] = {cat(gr.c0[0], gr.c0[1]), cat(gr.c0[2], gr.c0[3])};
+    h4 c1[S::H16], c0[S::H16];
+    color_dx<S>(T, lane, a, cdy, c1, c0);
     // colour L0^T for the logit inputs: dL/dlogit (fp16)
-    f4 cx = mfma32(TF(TC0 + 0), g0[0], z);
-    cx = mfma32(TF(TC0 + 1), g0[1], cx);
+    f4 cx = z;
+#pragma unroll
+    for (int kb = 0; kb < S::KB; kb++) cx = mfma32(TF(S::TC0 + kb), cat(c0[2 * kb], c0[2 * kb + 1]), cx);
     gr.cx = round_h4(cx);
     // glue: + d sigma on logit 0, clamped to the fp16 range, NaN -> 0
     h4 dd;
@@ -400,7 +446,7 @@ __device__ __forceinline__ void backward_tile(const h8* T, int lane, const Acts&
     // density L1^T: dX (64) masked by hd > 0 -> dY0
 #pragma unroll
     for (int mt = 0; mt < 4; mt++) {
-        const f4 d = mfma32(TF(TD1 + mt), gd1, z);
+        const f4 d = mfma32(TF(S::TD1 + mt), gd1, z);
         gr.d0[mt] = mask_h4(d, (mt & 1) ? hi4(a.hd[mt >> 1]) : lo4(a.hd[mt >> 1]));
     }
     if constexpr (FULL_DENC) {
@@ -408,30 +454,33 @@ __device__ __forceinline__ void backward_tile(const h8* T, int lane, const Acts&
         // density L0^T: dL/d(encoding)
 #pragma unroll
         for (int mt = 0; mt < 2; mt++) {
-            f4 d = mfma32(TF(TD0 + 2 * mt), gd0[0], z);
-            d = mfma32(TF(TD0 + 2 * mt + 1), gd0[1], d);
+            f4 d = mfma32(TF(S::TD0 + 2 * mt), gd0[0], z);
+            d = mfma32(TF(S::TD0 + 2 * mt + 1), gd0[1], d);
             gr.denc[mt] = round_h4(d);
         }
     }
 }
 
-__device__ __forceinline__ void load_weights(Weights& w, const h8* __restrict__ F, int lane)
+template <class S>
+__device__ __forceinline__ void load_weights(Weights<S>& w, const h8* __restrict__ F, int lane)
 {
 #pragma unroll
-    for (int f = 0; f < kFwdFrags; f++) w.F[f] = F[f * 64 + lane];
+    for (int f = 0; f < S::kFwdFrags; f++) w.F[f] = F[f * 64 + lane];
 }
 
-// biases into LDS (kBiasBlocks x 4 lane groups x f4)
+// biases into LDS (BLOCKS x 4 lane groups x f4)
+template <int BLOCKS>
 __device__ __forceinline__ void stage_bias(f4* sbias, const f4* __restrict__ bias)
 {
-    for (int e = threadIdx.x; e < kBiasBlocks * 4; e += blockDim.x) sbias[e] = bias[e];
+    for (int e = threadIdx.x; e < BLOCKS * 4; e += blockDim.x) sbias[e] = bias[e];
     __syncthreads();
 }
 
 // transposed fragments into LDS; the caller synchronises
+template <class S>
 __device__ __forceinline__ void stage_tr(h8* str, const h8* __restrict__ tr)
 {
-    for (int e = threadIdx.x; e < kTrFrags * 64; e += blockDim.x) str[e] = tr[e];
+    for (int e = threadIdx.x; e < S::kTrFrags * 64; e += blockDim.x) str[e] = tr[e];
 }
 
 __device__ __forceinline__ h8 load_cdy(const _Float16* __restrict__ cdy, int n, bool valid, int g)
@@ -476,14 +525,14 @@ struct FwdParams {
     _Float16* cin;    // nullable [N x 32]
 };
 
-template <int OUT_ACT>
+template <class S, int OUT_ACT>
 __global__ __launch_bounds__(256) void heads_fwd_kernel(const FwdParams p)
 {
-    __shared__ f4 sbias[kBiasBlocks * 4];
-    stage_bias(sbias, p.bias);
+    __shared__ f4 sbias[S::kBiasBlocks * 4];
+    stage_bias<S::kBiasBlocks>(sbias, p.bias);
     const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
-    Weights w;
-    load_weights(w, p.fwd, lane);
+    Weights<S> w;
+    load_weights<S>(w, p.fwd, lane);
     const int N = p.d_n ? min((int)*p.d_n, p.N) : p.N;
     const int ntiles = (N + 15) >> 4;
     const int nw = gridDim.x * (blockDim.x >> 6);
@@ -492,8 +541,8 @@ __global__ __launch_bounds__(256) void heads_fwd_kernel(const FwdParams p)
         const int n = tile * 16 + r;
         const bool valid = n < N;
         const TileIn in = load_tile(p.enc, p.plane, p.L, p.dirs, p.ray_idx, n, valid, g);
-        Acts a;
-        forward_tile(w, sbias, in, g, a);
+        Acts<S> a;
+        forward_tile<S>(w, sbias, in, g, a);
         if (!valid) continue;
         if (p.dout) {
             if (p.dout_full) *reinterpret_cast<f4*>(p.dout + (size_t)n * DOUT + 4 * g) = a.y;
@@ -534,8 +583,8 @@ struct DensityMaxParams {
 
 __global__ __launch_bounds__(256) void density_max_kernel(const DensityMaxParams p)
 {
-    __shared__ f4 sbias[kBiasBlocks * 4];
-    stage_bias(sbias, p.bias);
+    __shared__ f4 sbias[kDensityBiasBlocks * 4];
+    stage_bias<kDensityBiasBlocks>(sbias, p.bias);
     const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
     h8 F[6];
 #pragma unroll
@@ -592,7 +641,7 @@ struct BwdParams {
     _Float16* dloss;       // nullable [N x 16] density dL/dy
     _Float16* cdx;         // nullable [N x 32] colour dL/d(input): logit features, SH features 0
     float* ws_d;           // [gridDim.x][PD] (weight-gradient kernel)
-    float* ws_c;           // [gridDim.x][PC]
+    float* ws_c;           // [gridDim.x][S::PC]
     uint32_t* tile_live;   // nullable [tiles]: the dX kernel stores which tiles have a nonzero gradient, the
                            // weight-gradient kernel then visits only those
 };
@@ -649,15 +698,16 @@ __device__ __forceinline__ bool tile_live(h8 cdy, float ds, int g)
     return __ballot(mine) != 0ull;
 }
 
+template <class S>
 __global__ __launch_bounds__(256) void heads_dx_kernel(const BwdParams p)
 {
-    __shared__ f4 sbias[kBiasBlocks * 4];
-    __shared__ h8 str[kTrFrags * 64];
-    stage_tr(str, p.tr);
-    stage_bias(sbias, p.bias);
+    __shared__ f4 sbias[S::kBiasBlocks * 4];
+    __shared__ h8 str[S::kTrFrags * 64];
+    stage_tr<S>(str, p.tr);
+    stage_bias<S::kBiasBlocks>(sbias, p.bias);
     const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
-    Weights w;
-    load_weights(w, p.fwd, lane);
+    Weights<S> w;
+    load_weights<S>(w, p.fwd, lane);
     const int N = p.d_n ? min((int)*p.d_n, p.N) : p.N;
     const int ntiles = (N + 15) >> 4;
     const int nw = gridDim.x * (blockDim.x >> 6);
@@ -674,9 +724,9 @@ __global__ __launch_bounds__(256) void heads_dx_kernel(const BwdParams p)
         const bool live = tile_live(cur.cdy, cur.ds, g);
         if (p.tile_live && lane == 0) p.tile_live[tile] = live ? 1u : 0u;
         if (live) {
-            Acts a;
-            recompute_tile(w, sbias, cur.enc, cur.cin, g, a);
-            backward_tile<true>(str, lane, a, cur.cdy, cur.ds, gr);
+            Acts<S> a;
+            recompute_tile<S>(w, sbias, cur.enc, cur.cin, g, a);
+            backward_tile<S, true>(str, lane, a, cur.cdy, cur.ds, gr);
         } else {
             gr.denc[0] = gr.denc[1] = gr.cx = h4zero();
             gr.d1 = h4zero();
@@ -717,9 +767,10 @@ __device__ __forceinline__ f4 mfma16t(h4 a, h4 b, f4 c) { return __builtin_amdgc
 
 // Accumulators of the weight-gradient kernel, per head: dW blocks [out
 // block][in block] and db partials.
+template <class S>
 struct ColorAcc {
-    f4 c0[4][2], c1[4][4], c2[4];
-    float b0[4], b1[4], b2;
+    f4 c0[S::H16][2], c1[S::MID ? S::H16 : 1][S::H16], c2[S::H16];  // c1: with a middle layer only
+    float b0[S::H16], b1[S::H16], b2;
 };
 struct DensityAcc {
     f4 d0[4][2], d1[4];
@@ -729,7 +780,8 @@ struct DensityAcc {
 // The colour head's dW / db of one tile: dY2 = cdy, dY1 and dY0 from the
 // colour dX chain (backward_tile's operations, so the same bits); each
 // layer's update follows as soon as its dL/dy exists.
-__device__ __forceinline__ void color_dw_tile(ColorAcc& A, const h8* T, int lane, const Acts& a, h4 cdy, h4 ident)
+template <class S>
+__device__ __forceinline__ void color_dw_tile(ColorAcc<S>& A, const h8* T, int lane, const Acts<S>& a, h4 cdy, h4 ident)
 {
     const f4 z = f4zero();
     auto TF = [&](int q) { return T[q * 64 + lane]; };
@@ -737,29 +789,36 @@ __device__ __forceinline__ void color_dw_tile(ColorAcc& A, const h8* T, int lane
     {  // L2: cdy x h2
         const h4 Y = tblk(cdy, ident, &A.b2);
 #pragma unroll
-        for (int mi = 0; mi < 4; mi++) A.c2[mi] = mfma16t(Y, tblk(blk(a.h2, mi), ident), A.c2[mi]);
+        for (int mi = 0; mi < S::H16; mi++) A.c2[mi] = mfma16t(Y, tblk(blk(a.h2, mi), ident), A.c2[mi]);
     }
-    h4 c1[4];
+    h4 c1[S::H16];
 #pragma unroll
-    for (int mt = 0; mt < 4; mt++) c1[mt] = mask_h4(mfma32(TF(TC2 + mt), g2, z), blk(a.h2, mt));
-    {  // L1: dY1 x h1
-        h4 X[4];
+    for (int mt = 0; mt < S::H16; mt++) c1[mt] = mask_h4(mfma32(TF(S::TC2 + mt), g2, z), blk(a.h2, mt));
+    if constexpr (S::MID) {  // L1: dY1 x h1
+        h4 X[S::H16];
 #pragma unroll
-        for (int mi = 0; mi < 4; mi++) X[mi] = tblk(blk(a.h1, mi), ident);
+        for (int mi = 0; mi < S::H16; mi++) X[mi] = tblk(blk(a.h1, mi), ident);
 #pragma unroll
-        for (int mo = 0; mo < 4; mo++) {
+        for (int mo = 0; mo < S::H16; mo++) {
             const h4 Y = tblk(c1[mo], ident, &A.b1[mo]);
 #pragma unroll
-            for (int mi = 0; mi < 4; mi++) A.c1[mo][mi] = mfma16t(Y, X[mi], A.c1[mo][mi]);
+            for (int mi = 0; mi < S::H16; mi++) A.c1[mo][mi] = mfma16t(Y, X[mi], A.c1[mo][mi]);
         }
     }
-    const h8 g1[2] = {cat(c1[0], c1[1]), cat(c1[2], c1[3])};
+    h8 g1[S::KB];
+#pragma unroll
+    for (int kb = 0; kb < S::KB; kb++) g1[kb] = cat(c1[2 * kb], c1[2 * kb + 1]);
     const h4 X0 = tblk(lo4(a.cin), ident), X1 = tblk(hi4(a.cin), ident);
 #pragma unroll
-    for (int mo = 0; mo < 4; mo++) {  // L0: dY0 x cin
-        f4 d = mfma32(TF(TC1 + 2 * mo), g1[0], z);
-        d = mfma32(TF(TC1 + 2 * mo + 1), g1[1], d);
-        const h4 Y = tblk(mask_h4(d, blk(a.h1, mo)), ident, &A.b0[mo]);
+    for (int mo = 0; mo < S::H16; mo++) {  // L0: dY0 x cin
+        h4 y0 = c1[mo];
+        if constexpr (S::MID) {
+            f4 d = z;
+#pragma unroll
+            for (int kb = 0; kb < S::KB; kb++) d = mfma32(TF(S::TC1 + S::KB * mo + kb), g1[kb], d);
+            y0 = mask_h4(d, blk(a.h1, mo));
+        }
+        const h4 Y = tblk(y0, ident, &A.b0[mo]);
         A.c0[mo][0] = mfma16t(Y, X0, A.c0[mo][0]);
         A.c0[mo][1] = mfma16t(Y, X1, A.c0[mo][1]);
     }
@@ -767,6 +826,7 @@ __device__ __forceinline__ void color_dw_tile(ColorAcc& A, const h8* T, int lane
 
 // The density head's dW / db of one tile from its dL/dy (d1) and hidden
 // layer (hd): dY0 = (W1^T d1 masked by hd > 0), then the two updates.
+template <class S>
 __device__ __forceinline__ void density_dw_update(DensityAcc& A, const h8* T, int lane, const h8* hd, h8 enc, h4 d1,
                                                   h4 ident)
 {
@@ -774,7 +834,7 @@ __device__ __forceinline__ void density_dw_update(DensityAcc& A, const h8* T, in
     const h8 gd1 = cat(d1, h4zero());
     h4 d0[4];
 #pragma unroll
-    for (int mt = 0; mt < 4; mt++) d0[mt] = mask_h4(mfma32(T[(TD1 + mt) * 64 + lane], gd1, z), blk(hd, mt));
+    for (int mt = 0; mt < 4; mt++) d0[mt] = mask_h4(mfma32(T[(S::TD1 + mt) * 64 + lane], gd1, z), blk(hd, mt));
     {  // L1: dY1 x hd
         const h4 Y = tblk(d1, ident, &A.b1);
 #pragma unroll
@@ -791,12 +851,13 @@ __device__ __forceinline__ void density_dw_update(DensityAcc& A, const h8* T, in
 
 // The density head's dW / db of one tile when its dL/dy is not stored: the
 // whole dX chain down to it (backward_tile's operations, so the same bits).
-__device__ __forceinline__ void density_dw_tile(DensityAcc& A, const h8* T, int lane, const Acts& a, h4 cdy, float ds,
-                                                h4 ident)
+template <class S>
+__device__ __forceinline__ void density_dw_tile(DensityAcc& A, const h8* T, int lane, const Acts<S>& a, h4 cdy,
+                                                float ds, h4 ident)
 {
     Grads gr;
-    backward_tile<false>(T, lane, a, cat(cdy, h4zero()), ds, gr);
-    density_dw_update(A, T, lane, a.hd, a.enc, gr.d1, ident);
+    backward_tile<S, false>(T, lane, a, cat(cdy, h4zero()), ds, gr);
+    density_dw_update<S>(A, T, lane, a.hd, a.enc, gr.d1, ident);
 }
 
 // The density hidden layer of one tile (recompute_tile's operations for it)
@@ -877,19 +938,19 @@ struct LiveTiles {
 };
 
 // LIVE: p.tile_live holds the dX kernel's flags and only live tiles are visited
-template <bool LIVE>
+template <class S, bool LIVE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void heads_dw_kernel(const BwdParams p,
                                                                                                int color_blocks)
 {
-    __shared__ f4 sbias[kBiasBlocks * 4];
+    __shared__ f4 sbias[S::kBiasBlocks * 4];
     // the fragments during the tile loop, then the block partial of one head
     extern __shared__ __align__(16) unsigned char smem[];
     h8* str = reinterpret_cast<h8*>(smem);
-    h8* sfw = str + kTrFrags * 64;
+    h8* sfw = str + S::kTrFrags * 64;
     float* sred = reinterpret_cast<float*>(smem);
-    stage_tr(str, p.tr);
-    for (int e = threadIdx.x; e < kFwdFrags * 64; e += blockDim.x) sfw[e] = p.fwd[e];
-    stage_bias(sbias, p.bias);
+    stage_tr<S>(str, p.tr);
+    for (int e = threadIdx.x; e < S::kFwdFrags * 64; e += blockDim.x) sfw[e] = p.fwd[e];
+    stage_bias<S::kBiasBlocks>(sbias, p.bias);
     const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, wave = threadIdx.x >> 6;
     const int waves = blockDim.x >> 6;
     const LdsWeights w{{sfw, lane}};
@@ -902,12 +963,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void h
     const int N = p.d_n ? min((int)*p.d_n, p.N) : p.N;
     const int ntiles = (N + 15) >> 4;
     if (color) {
-        ColorAcc A;
+        ColorAcc<S> A;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < S::H16; i++) {
             A.c0[i][0] = A.c0[i][1] = A.c2[i] = f4zero();
+            if constexpr (S::MID) {
 #pragma unroll
-            for (int k = 0; k < 4; k++) A.c1[i][k] = f4zero();
+                for (int k = 0; k < S::H16; k++) A.c1[i][k] = f4zero();
+            }
             A.b0[i] = A.b1[i] = 0.f;
         }
         A.b2 = 0.f;
@@ -924,9 +987,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void h
                 reload_fence();
                 const int nt = lt.next();
                 const BwdIn nxt = load_bwd(p, nt * 16 + r, nt < ntiles && nt * 16 + r < N, g);
-                Acts a;
-                recompute_tile(w, sbias, in.enc, in.cin, g, a);
-                color_dw_tile(A, str, lane, a, lo4(in.cdy), ident);
+                Acts<S> a;
+                recompute_tile<S>(w, sbias, in.enc, in.cin, g, a);
+                color_dw_tile<S>(A, str, lane, a, lo4(in.cdy), ident);
                 in = nxt;
                 tile = nt;
             }
@@ -939,14 +1002,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void h
                 reload_fence();
                 const int nt = tile + stride;
                 const BwdIn nxt = load_bwd(p, nt * 16 + r, nt < ntiles && nt * 16 + r < N, g);
-                Acts a;
-                recompute_tile(w, sbias, in.enc, in.cin, g, a);
-                color_dw_tile(A, str, lane, a, lo4(in.cdy), ident);
+                Acts<S> a;
+                recompute_tile<S>(w, sbias, in.enc, in.cin, g, a);
+                color_dw_tile<S>(A, str, lane, a, lo4(in.cdy), ident);
                 in = nxt;
             }
         }
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < S::H16; i++) {
             A.b0[i] = gsum(A.b0[i]);
             A.b1[i] = gsum(A.b1[i]);
         }
@@ -956,20 +1019,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void h
             if (wave == wv) {
                 const bool first = wv == 0;
 #pragma unroll
-                for (int mo = 0; mo < 4; mo++) {
-                    put_w(sred, PC_W0, CIN, mo, 0, A.c0[mo][0], CHID, first, g, r);
-                    put_w(sred, PC_W0, CIN, mo, 1, A.c0[mo][1], CHID, first, g, r);
-                    put_b(sred, PC_B0, mo, A.b0[mo], CHID, first, g, r);
+                for (int mo = 0; mo < S::H16; mo++) {
+                    put_w(sred, S::PC_W0, CIN, mo, 0, A.c0[mo][0], S::CHID, first, g, r);
+                    put_w(sred, S::PC_W0, CIN, mo, 1, A.c0[mo][1], S::CHID, first, g, r);
+                    put_b(sred, S::PC_B0, mo, A.b0[mo], S::CHID, first, g, r);
+                    if constexpr (S::MID) {
 #pragma unroll
-                    for (int mi = 0; mi < 4; mi++) put_w(sred, PC_W1, CHID, mo, mi, A.c1[mo][mi], CHID, first, g, r);
-                    put_b(sred, PC_B1, mo, A.b1[mo], CHID, first, g, r);
-                    put_w(sred, PC_W2, CHID, 0, mo, A.c2[mo], COUT, first, g, r);
+                        for (int mi = 0; mi < S::H16; mi++)
+                            put_w(sred, S::PC_W1, S::CHID, mo, mi, A.c1[mo][mi], S::CHID, first, g, r);
+                        put_b(sred, S::PC_B1, mo, A.b1[mo], S::CHID, first, g, r);
+                    }
+                    put_w(sred, S::PC_W2, S::CHID, 0, mo, A.c2[mo], COUT, first, g, r);
                 }
-                put_b(sred, PC_B2, 0, A.b2, COUT, first, g, r);
+                put_b(sred, S::PC_B2, 0, A.b2, COUT, first, g, r);
             }
             __syncthreads();
         }
-        for (int e = threadIdx.x; e < PC; e += blockDim.x) p.ws_c[(size_t)rb * PC + e] = sred[e];
+        for (int e = threadIdx.x; e < S::PC; e += blockDim.x) p.ws_c[(size_t)rb * S::PC + e] = sred[e];
     } else {
         DensityAcc A;
 #pragma unroll
@@ -1004,7 +1070,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void h
                     load(nt, enc_n, d1_n);
                     h8 hd[2];
                     recompute_density(w, sbias, enc, g, hd);
-                    density_dw_update(A, str, lane, hd, enc, d1, ident);
+                    density_dw_update<S>(A, str, lane, hd, enc, d1, ident);
                     enc = enc_n;
                     d1 = d1_n;
                     t = nt;
@@ -1020,7 +1086,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void h
                     load(tile + stride, enc_n, d1_n);
                     h8 hd[2];
                     recompute_density(w, sbias, enc, g, hd);
-                    density_dw_update(A, str, lane, hd, enc, d1, ident);
+                    density_dw_update<S>(A, str, lane, hd, enc, d1, ident);
                     enc = enc_n;
                     d1 = d1_n;
                 }
@@ -1031,9 +1097,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void h
                 reload_fence();
                 const int nt = tile + stride;
                 const BwdIn nxt = load_bwd(p, nt * 16 + r, nt < ntiles && nt * 16 + r < N, g);
-                Acts a;
-                recompute_tile(w, sbias, in.enc, in.cin, g, a);
-                density_dw_tile(A, str, lane, a, lo4(in.cdy), in.ds, ident);
+                Acts<S> a;
+                recompute_tile<S>(w, sbias, in.enc, in.cin, g, a);
+                density_dw_tile<S>(A, str, lane, a, lo4(in.cdy), in.ds, ident);
                 in = nxt;
             }
         }
@@ -1061,8 +1127,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void h
 
 bool shapes_ok(const MlpShape& d, const MlpShape& c)
 {
-    return d.in == DIN && d.hid == DHID && d.out == DOUT && d.layers == 2 && c.in == CIN && c.hid == CHID &&
-           c.out == COUT && c.layers == 3;
+    return d.in == DIN && d.hid == DHID && d.out == DOUT && d.layers == 2 && c.in == CIN && c.out == COUT &&
+           (c.hid == 32 || c.hid == 64) && (c.layers == 2 || c.layers == 3);
 }
 
 int grid_for(const void* kern, int lds, int ntiles, int per_block_tiles)
@@ -1093,9 +1159,12 @@ void nerf_heads_pack(const NerfHeadsWeights& w, void* packed, hipStream_t s)
     p.fwd = reinterpret_cast<h8*>(base);
     p.tr = reinterpret_cast<h8*>(base + kFwdBytes);
     p.bias = reinterpret_cast<f4*>(base + kFwdBytes + kTrBytes);
-    const int threads = (kFwdFrags + kTrFrags) * 64 + kBiasBlocks * 4;
-    hipLaunchKernelGGL(pack_kernel, dim3((threads + 255) / 256), dim3(256), 0, s, p);
-    GRAFT_LAUNCH_CHECK();
+    with_head(w.color_hidden, w.color_layers, [&](auto head) {
+        using S = decltype(head);
+        const int threads = (S::kFwdFrags + S::kTrFrags) * 64 + S::kBiasBlocks * 4;
+        hipLaunchKernelGGL(pack_kernel<S>, dim3((threads + 255) / 256), dim3(256), 0, s, p);
+        GRAFT_LAUNCH_CHECK();
+    });
 }
 
 void nerf_heads_pack_density(const NerfHeadsWeights& w, void* packed, hipStream_t s)
@@ -1108,9 +1177,12 @@ void nerf_heads_pack_density(const NerfHeadsWeights& w, void* packed, hipStream_
     p.tr = reinterpret_cast<h8*>(base + kFwdBytes);
     p.bias = reinterpret_cast<f4*>(base + kFwdBytes + kTrBytes);
     p.density_only = true;
-    const int threads = (kFwdFrags + kTrFrags) * 64 + kBiasBlocks * 4;
-    hipLaunchKernelGGL(pack_kernel, dim3((threads + 255) / 256), dim3(256), 0, s, p);
-    GRAFT_LAUNCH_CHECK();
+    with_head(w.color_hidden, w.color_layers, [&](auto head) {
+        using S = decltype(head);
+        const int threads = (S::kFwdFrags + S::kTrFrags) * 64 + S::kBiasBlocks * 4;
+        hipLaunchKernelGGL(pack_kernel<S>, dim3((threads + 255) / 256), dim3(256), 0, s, p);
+        GRAFT_LAUNCH_CHECK();
+    });
 }
 
 void nerf_density_max(const NerfDensityMax& a, int N, hipStream_t s)
@@ -1162,11 +1234,12 @@ void nerf_heads_forward(const NerfHeadsFwd& a, int N, hipStream_t s, const uint3
     p.cout = a.color_out;
     p.cin = reinterpret_cast<_Float16*>(a.color_in);
     const int ntiles = (N + 15) / 16;
-    const void* kern = a.out_act == 1 ? (const void*)heads_fwd_kernel<1> : (const void*)heads_fwd_kernel<0>;
-    const int blocks = grid_for(kern, 0, ntiles, 4);
-    if (a.out_act == 1) hipLaunchKernelGGL(heads_fwd_kernel<1>, dim3(blocks), dim3(256), 0, s, p);
-    else hipLaunchKernelGGL(heads_fwd_kernel<0>, dim3(blocks), dim3(256), 0, s, p);
-    GRAFT_LAUNCH_CHECK();
+    with_head(a.color_hidden, a.color_layers, [&](auto head) {
+        using S = decltype(head);
+        const auto kern = a.out_act == 1 ? heads_fwd_kernel<S, 1> : heads_fwd_kernel<S, 0>;
+        hipLaunchKernelGGL(kern, dim3(grid_for((const void*)kern, 0, ntiles, 4)), dim3(256), 0, s, p);
+        GRAFT_LAUNCH_CHECK();
+    });
 }
 
 static BwdParams bwd_params(const NerfHeadsBwd& a, int N, const uint32_t* d_n)
@@ -1199,9 +1272,11 @@ void nerf_heads_dx(const NerfHeadsBwd& a, int N, hipStream_t s, const uint32_t* 
     if (N <= 0) return;
     const BwdParams p = bwd_params(a, N, d_n);
     const int ntiles = (N + 15) / 16;
-    const int blocks = grid_for((const void*)heads_dx_kernel, 0, ntiles, 4);
-    hipLaunchKernelGGL(heads_dx_kernel, dim3(blocks), dim3(256), 0, s, p);
-    GRAFT_LAUNCH_CHECK();
+    with_head(a.color_hidden, a.color_layers, [&](auto head) {
+        const auto kern = heads_dx_kernel<decltype(head)>;
+        hipLaunchKernelGGL(kern, dim3(grid_for((const void*)kern, 0, ntiles, 4)), dim3(256), 0, s, p);
+        GRAFT_LAUNCH_CHECK();
+    });
 }
 
 void nerf_heads_dw(const NerfHeadsBwd& a, const NerfHeadsGrads& out, int N, hipStream_t s, const uint32_t* d_n,
@@ -1210,19 +1285,22 @@ void nerf_heads_dw(const NerfHeadsBwd& a, const NerfHeadsGrads& out, int N, hipS
     // N = 0 still runs: the gradients are overwritten with zeros
     if (N < 0) return;
     BwdParams p = bwd_params(a, N, d_n);
-    const int lds = (int)std::max(kTrBytes + kFwdBytes, (size_t)PC * sizeof(float));
     const int per_head = a.dw_blocks > 0 ? a.dw_blocks : std::max(1, num_cus() / 2);
     // an even split also when the density dL/dy is stored (measured against
     // 70/30, 40/60 and 30/70 colour/density splits beside the scatter)
     const int cb = per_head, db = per_head;
-    Workspace& w = ws ? *ws : stream_workspace(s);
-    float* part = static_cast<float*>(w.get(((size_t)cb * PC + (size_t)db * PD) * sizeof(float)));
-    p.ws_c = part;
-    p.ws_d = part + (size_t)cb * PC;
-    if (p.tile_live) hipLaunchKernelGGL(heads_dw_kernel<true>, dim3(cb + db), dim3(256), lds, s, p, cb);
-    else hipLaunchKernelGGL(heads_dw_kernel<false>, dim3(cb + db), dim3(256), lds, s, p, cb);
-    GRAFT_LAUNCH_CHECK();
-    const MlpShape ds{DIN, DHID, DOUT, 2}, cs{CIN, CHID, COUT, 3};
+    with_head(a.color_hidden, a.color_layers, [&](auto head) {
+        using S = decltype(head);
+        const int lds = std::max((S::kTrFrags + S::kFwdFrags) * 64 * 16, std::max(S::PC, PD) * (int)sizeof(float));
+        Workspace& w = ws ? *ws : stream_workspace(s);
+        float* part = static_cast<float*>(w.get(((size_t)cb * S::PC + (size_t)db * PD) * sizeof(float)));
+        p.ws_c = part;
+        p.ws_d = part + (size_t)cb * S::PC;
+        const auto kern = p.tile_live ? heads_dw_kernel<S, true> : heads_dw_kernel<S, false>;
+        hipLaunchKernelGGL(kern, dim3(cb + db), dim3(256), lds, s, p, cb);
+        GRAFT_LAUNCH_CHECK();
+    });
+    const MlpShape ds{DIN, DHID, DOUT, 2}, cs{CIN, a.color_hidden, COUT, a.color_layers};
     mlp_grad_reduce(ds, p.ws_d, db, out.dW, out.dB, false, s);
     mlp_grad_reduce(cs, p.ws_c, cb, out.cW, out.cB, false, s);
 }
