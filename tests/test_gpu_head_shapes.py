@@ -1,0 +1,55 @@
+"""Training steps with the colour heads INerfTrainer (32 x 3) and InstantNerf's defaults (64 x 2) use, and the smallest
+one (32 x 2), replayed stage by stage on the oracle from the GPU's state before each step."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle"))
+
+import importlib  # noqa: E402
+
+import nerf_chain as nc  # noqa: E402
+from helpers import pkg  # noqa: E402
+
+scenes = importlib.import_module("3dmaker_amd.scenes")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("hidden,layers", [(32, 3), (64, 2), (32, 2)])
+def test_steps_match_oracle(hidden, layers):
+    print(f"[head shape] {hidden} x {layers}", flush=True)
+    P = pkg()
+    o = P.Nerf.default_options()
+    o.gridResolution[:] = [32, 32, 32]
+    o.aabbMin[:], o.aabbMax[:] = [-1.5] * 3, [1.5] * 3
+    o.hashTableSize, o.growthFactor = 1 << 14, 1.447
+    o.colorHiddenDim, o.colorNumLayers = hidden, layers
+    o.batchSize, o.rayChunkSize, o.renderBatchSize = 1 << 14, 4096, 1 << 14
+    o.beta2, o.epsilon, o.lossScale, o.lambdaDist, o.densityBias = 0.99, 1e-15, 128.0, 0.1, 0.0
+    nerf = P.Nerf(o)
+    nerf.set_keep_color_dx(True)
+    ro, rd = scenes.rays_c4(2048, n_cams=16, seed=4)
+    rng = np.random.default_rng(5)
+    gt = rng.random((2048, 3), dtype=np.float32)
+    lr, bg = 1e-2, (1.0, 1.0, 1.0)
+    nerf.set_learning_rate(lr)
+    nerf.set_bg_color(*bg)
+    first = 0
+    for _ in range(3):
+        st = nc.read_state(nerf, o)
+        march = nc.oracle_active(o, st, ro[first:], rd[first:])
+        R = int(march["active"])
+        assert R > 0 and int(march["total"]) > 0
+        sl = slice(first, first + R)
+        rgb = torch.zeros((R, 3), device="cuda")
+        dev = [torch.from_numpy(np.ascontiguousarray(a[sl])).cuda() for a in (ro, rd, gt)]
+        n, hits = nerf.train(dev[0], dev[1], dev[2], R, rgb_out=rgb)
+        torch.cuda.synchronize()
+        assert n == 1 and int(hits[0]) == int(march["total"])
+        nc.check_step(nerf, o, st, march, ro[sl], rd[sl], gt[sl], R, bg, lr, rgb.cpu().numpy())
+        first += R
+    nerf.close()
