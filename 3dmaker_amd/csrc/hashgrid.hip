@@ -246,7 +246,10 @@ void launch_encode(const GridMeta& m, const __half* table, const float* pos, int
 {
     GridKernelArgs a = grid_args(m, N, pos_stride);
     a.d_n = d_n;
-    const int tiles = std::min((N - 1) / kEncodeTile + 1, kEncodeTiles);
+    // With a count on the device N is only a bound, and each workgroup past the
+    // count costs its dispatch (about 350 per us): ordered samples, where the
+    // order of the levels does not matter, loop over at most 1,024 tiles then.
+    const int tiles = std::min((N - 1) / kEncodeTile + 1, d_n && !SCATTERED ? 1024 : kEncodeTiles);
     const int groups = (m.numLevels + kXcds - 1) / kXcds;
     hipLaunchKernelGGL((hash_encode_kernel<PLANAR, SCATTERED>), dim3(kXcds * tiles * (SCATTERED ? groups : 1)),
                        dim3(kEncodeTile), 0, stream, a, pos, reinterpret_cast<const _Float16*>(table),

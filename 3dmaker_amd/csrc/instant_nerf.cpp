@@ -134,6 +134,11 @@ struct NerfBuffers {
         __half* color_in = nullptr;    // [cap x 32]
         float* sigma = nullptr;
         float* rgb = nullptr;          // [cap x colour head width] (padded)
+        __half* enc = nullptr;         // [cap x 2L] level-major encodings of a round
+        uint32_t rays = 0;             // rays of one chunk of the rounds
+        graft::RenderSegments seg{};   // per ray of a chunk, and the rounds' counters
+        uint32_t* h_live = nullptr;    // pinned [kSegmentRounds + 1]: live rays after each round
+        hipEvent_t ev[2] = {};
         float3* dir = nullptr;         // one view direction (queryRadiance)
     } render;
     // model views
@@ -250,6 +255,20 @@ void InstantNerf::freeBuffers()
         dfree(b.render.sigma);
         dfree(b.render.rgb);
         dfree(b.render.dir);
+        dfree(b.render.enc);
+        dfree(b.render.seg.t);
+        dfree(b.render.seg.it);
+        dfree(b.render.seg.hits);
+        dfree(b.render.seg.pend);
+        dfree(b.render.seg.count);
+        dfree(b.render.seg.offset);
+        dfree(b.render.seg.acc);
+        dfree(b.render.seg.alive[0]);
+        dfree(b.render.seg.alive[1]);
+        dfree(b.render.seg.counters);
+        if (b.render.h_live) (void)hipHostFree(b.render.h_live);
+        for (hipEvent_t e : b.render.ev)
+            if (e) (void)hipEventDestroy(e);
         if (b.ev_fork) (void)hipEventDestroy(b.ev_fork);
         if (b.ev_join) (void)hipEventDestroy(b.ev_join);
         if (b.ev_done) (void)hipEventDestroy(b.ev_done);
@@ -1188,6 +1207,48 @@ void ensure_render(NerfBuffers& b, uint32_t cap, int color_width)
     b.render.cap = cap;
 }
 
+// What a front-to-back render of the hit batch `cap` keeps, on first use and
+// when the hit batch grows.
+void ensure_segments(NerfBuffers& b, uint32_t cap)
+{
+    NerfBuffers::Render& r = b.render;
+    const uint32_t rays = cap / graft::kSegmentLeast;
+    if (r.rays < rays) {
+        dfree(r.enc);
+        dfree(r.seg.t);
+        dfree(r.seg.it);
+        dfree(r.seg.hits);
+        dfree(r.seg.pend);
+        dfree(r.seg.count);
+        dfree(r.seg.offset);
+        dfree(r.seg.acc);
+        dfree(r.seg.alive[0]);
+        dfree(r.seg.alive[1]);
+        r.rays = 0;
+        r.enc = dalloc<__half>((size_t)2 * b.meta.numLevels * r.cap);
+        r.seg.t = dalloc<float>(rays);
+        r.seg.it = dalloc<int>(rays);
+        r.seg.hits = dalloc<uint32_t>(rays);
+        r.seg.pend = dalloc<float>(rays);
+        r.seg.count = dalloc<uint32_t>(rays);
+        r.seg.offset = dalloc<uint32_t>(rays);
+        r.seg.acc = dalloc<float4>(rays);
+        r.seg.alive[0] = dalloc<uint32_t>(rays);
+        r.seg.alive[1] = dalloc<uint32_t>(rays);
+        r.rays = rays;
+    }
+    if (!r.seg.counters) r.seg.counters = dalloc<uint32_t>(2 * graft::kSegmentRounds + 2);
+    if (!r.h_live)
+        GRAFT_HIP_CHECK(hipHostMalloc((void**)&r.h_live, (graft::kSegmentRounds + 1) * sizeof(uint32_t),
+                                      hipHostMallocDefault));
+    for (hipEvent_t& e : r.ev)
+        if (!e) GRAFT_HIP_CHECK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    r.seg.capacity = cap;
+    r.seg.sample_t = r.t;
+    r.seg.ray_idx = r.ray_idx;
+    r.seg.positions = r.positions;
+}
+
 }  // namespace
 
 uint32_t InstantNerf::renderHitBatch() const
@@ -1196,11 +1257,18 @@ uint32_t InstantNerf::renderHitBatch() const
     return (uint32_t)std::max(hb, MAX_HITS) & ~15u;
 }
 
-// renderImageHit (InstantNerf.cu:713-864): per chunk of rayChunkSize rays,
-// march once, then per hit batch: compaction from the first unrendered ray,
-// density inference, SH gather, colour inference, inference compositing
-// (compositing.cu:5-78) straight into d_rgb_out.  One host read per hit batch
-// (its active-ray count); the reference makes three blocking ones.
+// renderImageHit (InstantNerf.cu:713-864), front to back: a chunk of rays goes
+// through rounds of at most 32 samples per ray (march_segment), density, SH
+// gather and colour of the round's batch, and the inference compositing
+// (compositing.cu:5-78) carried on; rays leave at their last sample or below
+// T = 1e-4, where the compositing stops anyway, so that samples behind a
+// surface are neither marched nor evaluated and the sums are those of the
+// whole ray.  The live rays of a round are read a round later, while the next
+// one runs.  Of the 9.7 M samples of an 800 x 800 view of solid spheres 4 in 5
+// lie behind saturation.
+// With several samples per voxel (a round ends between voxels) or without an
+// output, whole rays per hit batch: compaction from the first unrendered ray,
+// one host read per hit batch; the reference makes three blocking ones.
 void InstantNerf::renderImageHit(const float3* d_rays_o, const float3* d_rays_d, uint32_t numRays, float* d_rgb_out,
                                  hipStream_t stream)
 {
@@ -1213,6 +1281,53 @@ void InstantNerf::renderImageHit(const float3* d_rays_o, const float3* d_rays_d,
     const graft::MlpShape dshape{2 * o.numLevels, db.hw.hiddenDim, db.hw.outputDim, db.hw.numLayers};
     const graft::MlpShape cshape = shape_of(cb.hw);
     ensure_render(b, hitBatch, cshape.out);
+    if (o.samplesPerVoxel == 1 && d_rgb_out) {
+        ensure_segments(b, hitBatch);
+        const graft::RenderSegments& seg = b.render.seg;
+        const graft::OccGrid g = occ_grid(o, d_occupancyGrid);
+        const uint32_t chunk = hitBatch / graft::kSegmentLeast;
+        graft::NerfFwdArgs fa;
+        fa.dshape = dshape;
+        fa.pos = reinterpret_cast<const float*>(b.render.positions);
+        fa.pos_stride = 4;
+        fa.table = db.fwd_hashtable;
+        fa.meta = &b.meta;
+        fa.dW = db.fwd_weights;
+        fa.dB = db.master_biases;
+        fa.ray_idx = b.render.ray_idx;
+        fa.density_bias = o.densityBias;
+        fa.sigma = b.render.sigma;
+        fa.cshape = cshape;
+        fa.out_act = cb.hw.outputActivation;
+        fa.cW = cb.fwd_weights;
+        fa.cB = cb.master_biases;
+        fa.color_out = b.render.rgb;
+        fa.enc_scratch = b.render.enc;
+        fa.enc_plane = (int)hitBatch;
+        fa.heads_packed = b.heads_packed;  // repacked here: the weights may have been loaded or changed
+        for (uint32_t c0 = 0; c0 < numRays; c0 += chunk) {
+            const uint32_t R = std::min(chunk, numRays - c0);
+            const float3* co = d_rays_o + c0;
+            const float3* cd = d_rays_d + c0;
+            fa.dirs = cd;
+            graft::clear_segment_counters(seg, stream);
+            for (uint32_t round = 0; round < (uint32_t)graft::kSegmentRounds; round++) {
+                graft::march_segment(seg, R, round, co, cd, g, stream);
+                graft::nerf_forward(fa, (int)hitBatch, stream, seg.counters + 2 * round + 1);
+                fa.heads_prepacked = true;
+                graft::composite_segment(seg, R, round, b.render.sigma, b.render.rgb, cshape.out, o.bgColor,
+                                         d_rgb_out + (size_t)c0 * 3, stream);
+                GRAFT_HIP_CHECK(hipMemcpyAsync(b.render.h_live + round, seg.counters + 2 * (round + 1), sizeof(uint32_t),
+                                               hipMemcpyDeviceToHost, stream));
+                GRAFT_HIP_CHECK(hipEventRecord(b.render.ev[round & 1], stream));
+                if (round > 0) {
+                    GRAFT_HIP_CHECK(hipEventSynchronize(b.render.ev[(round - 1) & 1]));
+                    if (b.render.h_live[round - 1] == 0) break;
+                }
+            }
+        }
+        return;
+    }
     const graft::OccGrid g = occ_grid(o, d_occupancyGrid);
     StepSet& S = b.set[0];  // the render path runs on the caller's stream only
     const uint32_t* d_rays = S.result;

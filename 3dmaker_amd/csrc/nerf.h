@@ -60,6 +60,41 @@ void march_compact_stored(uint32_t R, const float3* o, const float3* d, const Oc
                           float* t_out, uint32_t* ray_idx, float4* pos_out, const MarchScratch& scratch,
                           hipStream_t s, uint32_t* counts_out = nullptr);
 
+// A front-to-back render of R rays (R * kSegmentLeast <= capacity): rounds of
+// march_segment, the network on the batch, composite_segment, until no ray is
+// alive.  A ray ends at its last sample or where its transmittance falls below
+// 1e-4, so that nothing behind that is marched or evaluated.  One sample per
+// voxel (samplesPerVoxel 1).  counters: round r starts with counters[2 r] live
+// rays (round 0: R) and has counters[2 r + 1] samples; all zero before round 0.
+constexpr int kSegmentLeast = 8, kSegmentMost = 32;
+constexpr int kSegmentRounds = kMaxHits / kSegmentLeast + 2;
+constexpr uint32_t kSegmentLast = 0x80000000u;  // in count: no sample behind this round's
+struct RenderSegments {
+    // per ray
+    float* t;
+    int* it;
+    uint32_t* hits;
+    float* pend;
+    uint32_t* count;
+    uint32_t* offset;
+    float4* acc;            // colour and transmittance so far
+    uint32_t* alive[2];     // live rays of even and odd rounds
+    // per sample of a round
+    uint32_t capacity;
+    float* sample_t;
+    uint32_t* ray_idx;
+    float4* positions;
+    uint32_t* counters;     // [2 kSegmentRounds + 2]
+};
+void march_segment(const RenderSegments& seg, uint32_t R, uint32_t round, const float3* o, const float3* d,
+                   const OccGrid& g, hipStream_t s);
+void clear_segment_counters(const RenderSegments& seg, hipStream_t s);
+// composite_infer's operations on the round's samples, carried on from round to
+// round; a ray that ends writes its colour to rgb_out [R x 3], the others are
+// the live rays of the next round.
+void composite_segment(const RenderSegments& seg, uint32_t R, uint32_t round, const float* sigma, const float* rgb,
+                       int rgb_stride, float3 bg, float* rgb_out, hipStream_t s);
+
 // march_rays_dda_calc_hits (processRays.cu:626-737): per-ray sample counts only.
 void march_count(uint32_t R, const float3* o, const float3* d, const float3* d_inv, const float* nears,
                  const float* fars, const OccGrid& g, int K, uint32_t* counts, hipStream_t s);

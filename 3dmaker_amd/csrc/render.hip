@@ -188,6 +188,64 @@ __global__ __launch_bounds__(256) void composite_infer_kernel(const CompositeArg
     }
 }
 
+__global__ __launch_bounds__(256) void clear_counters_kernel(uint32_t* counters, int n)
+{
+    for (int i = threadIdx.x; i < n; i += 256) counters[i] = 0u;
+}
+
+// composite_infer_kernel's operations in its order, one round's samples at a
+// time: one thread per live ray.
+__global__ __launch_bounds__(256) void composite_segment_kernel(const RenderSegments s, uint32_t R, uint32_t round,
+                                                                const float* __restrict__ sigma,
+                                                                const float* __restrict__ rgb, int rgb_stride,
+                                                                float3 bg, float* __restrict__ out)
+{
+    const uint32_t live = round == 0 ? R : s.counters[2 * round];
+    const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+    if (blockIdx.x * 256 >= live) return;
+    bool on = false;
+    uint32_t ray = 0;
+    if (i < live) {
+        ray = round == 0 ? i : s.alive[round & 1][i];
+        const uint32_t word = s.count[ray], n = word & ~kSegmentLast, off = s.offset[ray];
+        const bool last = (word & kSegmentLast) != 0u;
+        float4 a = round == 0 ? make_float4(0.0f, 0.0f, 0.0f, 1.0f) : s.acc[ray];
+        bool done = false;
+        for (uint32_t k = 0; k < n; k++) {
+            const uint32_t idx = off + k;
+            const float t = s.sample_t[idx];
+            float delta = k + 1 < n ? s.sample_t[idx + 1] - t : last ? 1e-3f : s.pend[ray] - t;
+            if (delta < 0.0f) delta = 0.0f;
+            const float alpha = 1.0f - nerf_expf(-sigma[idx] * delta);
+            const float w = alpha * a.w;
+            const float* c = rgb + (size_t)rgb_stride * idx;
+            a.x += w * c[0];
+            a.y += w * c[1];
+            a.z += w * c[2];
+            a.w *= (1.0f - alpha);
+            if (a.w < 1e-4f) {
+                done = true;
+                break;
+            }
+        }
+        if (done || last) {
+            out[3 * (size_t)ray] = a.x + a.w * bg.x;
+            out[3 * (size_t)ray + 1] = a.y + a.w * bg.y;
+            out[3 * (size_t)ray + 2] = a.z + a.w * bg.z;
+        } else {
+            s.acc[ray] = a;
+            on = true;
+        }
+    }
+    const uint64_t m = __ballot(on);
+    if (m == 0ull) return;
+    const int lane = threadIdx.x & 63;
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(&s.counters[2 * (round + 1)], (uint32_t)__popcll(m));
+    base = __shfl(base, 0, 64);
+    if (on) s.alive[(round + 1) & 1][base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull))] = ray;
+}
+
 __global__ __launch_bounds__(256) void color_grad_kernel(const ColorGradArgs a, const uint32_t* __restrict__ d_rays,
                                                          uint32_t rays_max)
 {
@@ -827,6 +885,21 @@ void composite_infer(const CompositeArgs& a, uint32_t base, uint32_t rays_done, 
     if (rays_max == 0) return;
     hipLaunchKernelGGL(composite_infer_kernel, dim3(blocks_for(rays_max)), dim3(256), 0, s, a, base, rays_done,
                        d_rays, rays_max);
+    GRAFT_LAUNCH_CHECK();
+}
+
+void clear_segment_counters(const RenderSegments& seg, hipStream_t s)
+{
+    hipLaunchKernelGGL(clear_counters_kernel, dim3(1), dim3(256), 0, s, seg.counters, 2 * kSegmentRounds + 2);
+    GRAFT_LAUNCH_CHECK();
+}
+
+void composite_segment(const RenderSegments& seg, uint32_t R, uint32_t round, const float* sigma, const float* rgb,
+                       int rgb_stride, float3 bg, float* rgb_out, hipStream_t s)
+{
+    if (R == 0) return;
+    hipLaunchKernelGGL(composite_segment_kernel, dim3((R + 255) / 256), dim3(256), 0, s, seg, R, round, sigma, rgb,
+                       rgb_stride, bg, rgb_out);
     GRAFT_LAUNCH_CHECK();
 }
 

@@ -1,0 +1,82 @@
+"""The front-to-back render against one whole-ray evaluation of the same rays: samples by the march launcher, the
+heads' own kernels and the oracle's inference compositing.  Rays with one to hundreds of samples, thin and opaque
+fields, chunks of rays larger than a hit batch holds, none, one and odd ray counts."""
+import os
+import sys
+
+import numpy as np
+import pytest
+
+torch = pytest.importorskip("torch")
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "oracle"))
+import pyoracle as orc  # noqa: E402
+
+import importlib  # noqa: E402
+
+from helpers import assert_close, pkg  # noqa: E402
+
+scenes = importlib.import_module("3dmaker_amd.scenes")
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("R,batch,cascades,bias,hidden,layers", [
+    (1, 1 << 14, 1, 0.0, 64, 3),        # one ray
+    (2047, 1 << 14, 1, 4.0, 32, 3),     # thin field: no ray saturates, many rounds
+    (5000, 1 << 14, 1, -6.0, 64, 2),    # opaque field: most rays end in the first round; several chunks of rays
+    (777, 1 << 12, 3, 1.0, 64, 4),      # cascades; a colour head outside the MFMA kernels' shapes
+])
+def test_render_matches_whole_rays(R, batch, cascades, bias, hidden, layers):
+    print(f"[render rounds] R={R} batch={batch} C={cascades} bias={bias} colour {hidden} x {layers}", flush=True)
+    P = pkg()
+    res, mips, T_ = 64, 4, 1 << 14
+    o = P.Nerf.default_options()
+    o.gridResolution[:] = [res] * 3
+    o.aabbMin[:], o.aabbMax[:] = [-1.5] * 3, [1.5] * 3
+    o.levelsMipmap, o.numCascades, o.samplesPerVoxel = mips, cascades, 1
+    o.hashTableSize, o.growthFactor = T_, 1.447
+    o.colorHiddenDim, o.colorNumLayers = hidden, layers
+    o.batchSize, o.rayChunkSize, o.renderBatchSize = batch, 1024, batch
+    o.densityBias = bias
+    o.bgColor[:] = [0.25, 0.5, 1.0]
+    nerf = P.Nerf(o)
+    rng = np.random.default_rng(3)
+    table = rng.normal(0, 0.5, 16 * T_ * 2).astype(np.float32)
+    nerf.density.load_hashgrid(table)
+    l0 = [rng.random((res, res, res)) < (0.5 if c == 0 else 0.02) for c in range(cascades)]
+    bits = scenes.pack_grid(l0, mips)
+    nerf.set_occupancy(bits)
+    nerf.set_memory_mode(True)
+    ro, rd = scenes.rays_c4(R, n_cams=8, seed=6)
+    d_o, d_d = torch.from_numpy(ro).cuda(), torch.from_numpy(rd).cuda()
+    rgb = torch.full((R, 3), -1.0, device="cuda")
+    nerf.render(d_o, d_d, R, rgb)
+    rgb2 = torch.full((R, 3), -1.0, device="cuda")
+    nerf.render(d_o, d_d, R, rgb2)
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(rgb.cpu().numpy(), rgb2.cpu().numpy())
+
+    mn, mx = np.float32([-1.5] * 3), np.float32([1.5] * 3)
+    di, near, far = orc.ray_aabb_inv(ro, rd, mn, mx, cascades)
+    m = orc.march_hits(ro, rd, di, near, far, bits, [res] * 3, mn, mx, cascades, mips, 1, 1 << 24)
+    N = int(m["total"])
+    cnt, off, t, ridx = m["counts"][:R], m["offsets"][:R], m["t"][:N], m["ray_idx"][:N]
+    assert N > 0 or R == 1
+    def weights(net, i, h, out, n):
+        W = np.zeros(sum((out if l == n - 1 else h) * (i if l == 0 else h) for l in range(n)), np.float32)
+        B = np.zeros(sum(out if l == n - 1 else h for l in range(n)), np.float32)
+        net.save_weights(W, B)
+        return W.astype(np.float16), B
+
+    dW, dB = weights(nerf.density, 32, 64, 16, 2)
+    cW, cB = weights(nerf.color, 32, hidden, 8, layers)
+    enc = orc.hash_encode(np.ascontiguousarray(m["pos"][:N]), table.astype(np.float16), T_, 16, 16, 1.447)
+    y, _ = orc.mlp_forward(enc, dW, dB, 32, 64, 16, 2, save_acts=False)
+    cin, sig = orc.sh_gather(rd, ridx, y, bias)
+    c, _ = orc.mlp_forward(cin, cW, cB, 32, hidden, 8, layers, out_act=1, save_acts=False)
+    want = orc.composite_infer(off, cnt, t, sig, np.ascontiguousarray(c[:, :3]), np.float32([0.25, 0.5, 1.0]))
+    want = want["rgb"] if isinstance(want, dict) else want[0]
+    assert_close(rgb.cpu().numpy(), want, what="rgb")
+    if cascades == 1 and R > 1:
+        assert cnt.max() > 17  # more than one round
+    nerf.close()
