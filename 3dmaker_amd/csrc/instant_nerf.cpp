@@ -1281,6 +1281,9 @@ void InstantNerf::renderImageHit(const float3* d_rays_o, const float3* d_rays_d,
     const graft::MlpShape dshape{2 * o.numLevels, db.hw.hiddenDim, db.hw.outputDim, db.hw.numLayers};
     const graft::MlpShape cshape = shape_of(cb.hw);
     ensure_render(b, hitBatch, cshape.out);
+    // a render discards the prefetched rays; its whole-ray form also reuses the march store and step set 0
+    b.ms[0].version = b.ms[1].version = -1;
+    b.pre.valid = false;
     if (o.samplesPerVoxel == 1 && d_rgb_out) {
         ensure_segments(b, hitBatch);
         const graft::RenderSegments& seg = b.render.seg;
@@ -1333,8 +1336,6 @@ void InstantNerf::renderImageHit(const float3* d_rays_o, const float3* d_rays_d,
     const uint32_t* d_rays = S.result;
     const uint32_t* d_hits = S.result + 1;
     MarchStore& M = b.ms[b.cur];
-    b.ms[0].version = b.ms[1].version = -1;  // the march store is reused below
-    b.pre.valid = false;                     // and so is step set 0
 
     for (uint32_t c0 = 0; c0 < numRays; c0 += (uint32_t)o.rayChunkSize) {
         const uint32_t R = std::min<uint32_t>((uint32_t)o.rayChunkSize, numRays - c0);
