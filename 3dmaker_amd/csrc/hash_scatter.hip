@@ -108,6 +108,8 @@ struct ScatterArgs {
     uint32_t mask;
     uint32_t chunk;  // records per accumulate chunk of a split bin
     uint32_t split;  // bins of more records are split into chunks
+    uint32_t late;   // bins of one chunk left to the accumulate's second phase
+    int lpg;         // levels per workgroup of the count and distribute passes (blockIdx.y: their group)
     float scale[kMaxLevels];
     int res[kMaxLevels];
     int bin_base[kMaxLevels + 1];   // bins of level l: [bin_base[l], bin_base[l + 1])
@@ -177,26 +179,26 @@ __device__ __forceinline__ int sample_count(const ScatterArgs& a) { return a.d_n
 // |dL/denc| of a level's feature pair: the larger fp16 magnitude, as bits.
 __device__ __forceinline__ uint32_t pair_mag(uint32_t gb) { return max(gb & 0x7fffu, (gb >> 16) & 0x7fffu); }
 
-// dL/denc of levels [l0, l0 + kLevelGroup) of one sample's row, loaded
-// together (16-byte loads when the row is 16-byte aligned); zero past L.
+// dL/denc of levels [l0, l1) of one sample's row, at most kLevelGroup, loaded
+// together (16-byte loads when the row and l0 are 16-byte aligned); zero from
+// l1 on.
 constexpr int kLevelGroup = 16;
 
-__device__ __forceinline__ void load_levels(const uint32_t* grow, int l0, int L, bool vec,
+__device__ __forceinline__ void load_levels(const uint32_t* grow, int l0, int l1, bool vec,
                                             uint32_t (&g)[kLevelGroup])
 {
-    if (vec && l0 + kLevelGroup <= L) {
-        const uint4* v = reinterpret_cast<const uint4*>(grow + l0);
 #pragma unroll
-        for (int j = 0; j < kLevelGroup / 4; j++) {
-            const uint4 t = v[j];
-            g[4 * j] = t.x;
-            g[4 * j + 1] = t.y;
-            g[4 * j + 2] = t.z;
-            g[4 * j + 3] = t.w;
+    for (int j = 0; j < kLevelGroup; j += 4) {
+        if (vec && l0 + j + 4 <= l1) {
+            const uint4 t = *reinterpret_cast<const uint4*>(grow + l0 + j);
+            g[j] = t.x;
+            g[j + 1] = t.y;
+            g[j + 2] = t.z;
+            g[j + 3] = t.w;
+        } else {
+#pragma unroll
+            for (int k = j; k < j + 4; k++) g[k] = l0 + k < l1 ? grow[l0 + k] : 0u;
         }
-    } else {
-#pragma unroll
-        for (int j = 0; j < kLevelGroup; j++) g[j] = l0 + j < L ? grow[l0 + j] : 0u;
     }
 }
 
@@ -239,10 +241,13 @@ __global__ __launch_bounds__(kBinThreads) void scatter_count_kernel(const Scatte
     extern __shared__ uint32_t sh[];
     uint32_t* hist = sh;
     uint32_t* lmax = sh + a.bins;
-    for (int i = threadIdx.x; i < a.bins + a.L; i += kBinThreads) sh[i] = 0u;
+    const int lo = blockIdx.y * a.lpg, hi = min(lo + a.lpg, a.L);  // this workgroup's levels
+    const int b0 = a.bin_base[lo], b1 = a.bin_base[hi];            // and bins
+    for (int i = b0 + (int)threadIdx.x; i < b1; i += kBinThreads) hist[i] = 0u;
+    for (int i = lo + (int)threadIdx.x; i < hi; i += kBinThreads) lmax[i] = 0u;
     __syncthreads();
     const int N = sample_count(a);
-    const bool vec = (a.L & 3) == 0;
+    const bool vec = ((a.L | a.lpg) & 3) == 0 && (reinterpret_cast<uintptr_t>(denc) & 15) == 0;
     for (int k = 0; k < kSamplesPerThread; k++) {
         const int n = blockIdx.x * kRound + k * kBinThreads + threadIdx.x;
         const bool valid = n < N && (!a.tile_live || a.tile_live[n >> 4] != 0u);
@@ -254,13 +259,13 @@ __global__ __launch_bounds__(kBinThreads) void scatter_count_kernel(const Scatte
             py = pp[1];
             pz = pp[2];
         }
-        for (int l0 = 0; l0 < a.L; l0 += kLevelGroup) {
+        for (int l0 = lo; l0 < hi; l0 += kLevelGroup) {
             uint32_t gv[kLevelGroup];
-            load_levels(grow, l0, a.L, vec, gv);
+            load_levels(grow, l0, hi, vec, gv);
 #pragma unroll
             for (int j = 0; j < kLevelGroup; j++) {
                 const int l = l0 + j;
-                if (l >= a.L) break;
+                if (l >= hi) break;
                 const uint32_t gb = valid ? gv[j] : 0u;
                 const bool live = (gb & 0x7fff7fffu) != 0u;  // else both features +-0: no product is nonzero
                 const uint32_t m = __ockl_wfred_max_u32(pair_mag(gb));
@@ -279,8 +284,8 @@ __global__ __launch_bounds__(kBinThreads) void scatter_count_kernel(const Scatte
         }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < a.bins; i += kBinThreads) counts[(size_t)blockIdx.x * a.bins + i] = hist[i];
-    for (int i = threadIdx.x; i < a.L; i += kBinThreads) lvlmax[(size_t)blockIdx.x * a.L + i] = lmax[i];
+    for (int i = b0 + (int)threadIdx.x; i < b1; i += kBinThreads) counts[(size_t)blockIdx.x * a.bins + i] = hist[i];
+    for (int i = lo + (int)threadIdx.x; i < hi; i += kBinThreads) lvlmax[(size_t)blockIdx.x * a.L + i] = lmax[i];
 }
 
 // Block x: bins [64 x, 64 x + 64), one per lane, and kPrefixWaves waves, each
@@ -425,7 +430,7 @@ __global__ __launch_bounds__(kBinThreads) void scatter_distribute_kernel(
     __shared__ uint32_t wsum[kBinThreads / 64];
     __shared__ uint64_t wsum64[kBinThreads / 64];
     block_exclusive_scan(totals, cur, a.bins, wsum);
-    if (blockIdx.x == 0) {
+    if (blockIdx.x == 0 && blockIdx.y == 0) {
         const uint32_t C = a.chunk, S = a.split;
         // per bin, four counters packed in one word and scanned together (no
         // field's total carries into the next: chunks of split bins < 2^18,
@@ -463,15 +468,17 @@ __global__ __launch_bounds__(kBinThreads) void scatter_distribute_kernel(
         }
         if (threadIdx.x == 0) {
             const uint32_t all = nsplit + nlarge + nsmall;
-            nchunks[0] = all - min(nsmall, kLateChunks);
+            nchunks[0] = all - min(nsmall, a.late);
             nchunks[1] = nmerge;
             nchunks[2] = all;
         }
     }
-    for (int b = threadIdx.x; b < a.bins; b += kBinThreads) cur[b] += prefix[(size_t)blockIdx.x * a.bins + b];
+    const int lo = blockIdx.y * a.lpg, hi = min(lo + a.lpg, a.L);
+    for (int b = a.bin_base[lo] + (int)threadIdx.x; b < a.bin_base[hi]; b += kBinThreads)
+        cur[b] += prefix[(size_t)blockIdx.x * a.bins + b];
     __syncthreads();
     const int N = sample_count(a);
-    const bool vec = (a.L & 3) == 0;
+    const bool vec = ((a.L | a.lpg) & 3) == 0 && (reinterpret_cast<uintptr_t>(denc) & 15) == 0;
     for (int k = 0; k < kSamplesPerThread; k++) {
         const int n = blockIdx.x * kRound + k * kBinThreads + threadIdx.x;
         if (n >= N) break;
@@ -479,13 +486,13 @@ __global__ __launch_bounds__(kBinThreads) void scatter_distribute_kernel(
         const float* pp = pos + (size_t)n * a.pos_stride;
         const float px = pp[0], py = pp[1], pz = pp[2];
         const uint32_t* grow = reinterpret_cast<const uint32_t*>(denc + (size_t)n * 2 * a.L);
-        for (int l0 = 0; l0 < a.L; l0 += kLevelGroup) {
+        for (int l0 = lo; l0 < hi; l0 += kLevelGroup) {
             uint32_t gv[kLevelGroup];
-            load_levels(grow, l0, a.L, vec, gv);
+            load_levels(grow, l0, hi, vec, gv);
 #pragma unroll
             for (int j = 0; j < kLevelGroup; j++) {
                 const int l = l0 + j;
-                if (l >= a.L) break;
+                if (l >= hi) break;
                 const uint32_t gb = gv[j];
                 if ((gb & 0x7fff7fffu) == 0u) continue;
                 Pairs p;
@@ -1163,7 +1170,8 @@ __device__ __forceinline__ void do_merge(SliceLds<ADAM>& S, const ScatterArgs& a
 // bins of one chunk.  Phase 2 (after phase 1: the kernel boundary orders the
 // partial slices, no device-scope fence or counter is needed): the merges of
 // the bins of several chunks, beside the last bins of one chunk (chunks
-// [nchunks[0], nchunks[2])), so that the merges run on a busy GPU.  Two
+// [nchunks[0], nchunks[2])), so that the merges run on a busy GPU.  A batch
+// too small for a split bin leaves nothing to phase 2.  Two
 // blocks per CU (the LDS holds two slices): at most 128 VGPRs.
 template <bool ADAM, bool PHASE2>
 __global__ __launch_bounds__(kAccThreads) __attribute__((amdgpu_waves_per_eu(4))) void scatter_accumulate_kernel(
@@ -1358,6 +1366,23 @@ int scatter_plan_max_samples(const ScatterPlan* p) { return p ? p->maxN : 0; }
 
 namespace {
 
+// The level groups (blockIdx.y) of the count and distribute passes, and
+// a.lpg.  A workgroup walks its 512 samples through its levels one after the
+// other, a chain of LDS atomics per level, so a small batch (few rounds) is
+// bound by that chain and cuts the levels over enough workgroups for one per
+// CU: a training step of 4096 points 103 -> 75 us (with the single accumulate
+// launch below); with 8 or 4 levels per workgroup instead of one 87 and 81.  From
+// 256 rounds on the GPU is full and a round keeps all its levels: with two
+// groups at 2^18 samples every row of dL/denc is fetched twice, a training
+// step over rays 3 % slower, a stand-alone scatter of ray samples 4 % faster.
+int level_groups(ScatterArgs& a)
+{
+    const int want = a.rounds < 256 ? 256 / a.rounds : 1;
+    a.lpg = a.L;
+    for (int lpg = kLevelGroup / 2; lpg >= 1 && (a.L + a.lpg - 1) / a.lpg < want; lpg /= 2) a.lpg = std::min(lpg, a.L);
+    return (a.L + a.lpg - 1) / a.lpg;
+}
+
 // count, prefix, distribute, then (after wait_before, when given) accumulate:
 // into grads, or (ta) as the fused table update.
 void scatter_launch(ScatterPlan* p, const GridMeta& m, const __half* denc, const float* pos, int pos_stride,
@@ -1376,10 +1401,16 @@ void scatter_launch(ScatterPlan* p, const GridMeta& m, const __half* denc, const
     a.N = N;
     a.pos_stride = pos_stride;
     a.rounds = (N + kRound - 1) / kRound;
+    const int groups = level_groups(a);
+    // a sample has at most 4 records in a bin: without a bin to split there is
+    // no merge, and the second phase's launch (10 us of mostly empty
+    // workgroups at 4096 samples) is left out
+    const bool one_phase = 4ull * (unsigned long long)N <= a.split;
+    a.late = one_phase ? 0u : kLateChunks;
     const auto* dh = reinterpret_cast<const _Float16*>(denc);
     const size_t lds_count = (size_t)(a.bins + a.L) * 4;
     const size_t lds_dist = (size_t)(((a.bins + 1) & ~1) + 2 * a.bins) * 4;
-    hipLaunchKernelGGL(scatter_count_kernel, dim3(a.rounds), dim3(kBinThreads), lds_count, stream, a, pos, dh,
+    hipLaunchKernelGGL(scatter_count_kernel, dim3(a.rounds, groups), dim3(kBinThreads), lds_count, stream, a, pos, dh,
                        p->counts, p->lvlmax);
     GRAFT_LAUNCH_CHECK();
     const int prefix_blocks = std::max((a.bins + kPrefixBins - 1) / kPrefixBins, a.L);
@@ -1387,7 +1418,7 @@ void scatter_launch(ScatterPlan* p, const GridMeta& m, const __half* denc, const
                        p->lvlmax, p->lvlmax_final);
     GRAFT_LAUNCH_CHECK();
     const uint32_t cap = (uint32_t)(4ull * (unsigned long long)a.L * (unsigned long long)p->maxN);
-    hipLaunchKernelGGL(scatter_distribute_kernel, dim3(a.rounds), dim3(kBinThreads), lds_dist, stream, a, pos, dh,
+    hipLaunchKernelGGL(scatter_distribute_kernel, dim3(a.rounds, groups), dim3(kBinThreads), lds_dist, stream, a, pos, dh,
                        p->counts, p->totals, p->rec, cap, p->chunks, p->merges, p->nchunks);
     GRAFT_LAUNCH_CHECK();
     if (wait_before) GRAFT_HIP_CHECK(hipStreamWaitEvent(stream, wait_before, 0));
@@ -1401,12 +1432,14 @@ void scatter_launch(ScatterPlan* p, const GridMeta& m, const __half* denc, const
         hipLaunchKernelGGL((scatter_accumulate_kernel<true, false>), dim3(grid), dim3(kAccThreads), 0, stream, a, g,
                            *ta);
         GRAFT_LAUNCH_CHECK();
+        if (one_phase) return;
         hipLaunchKernelGGL((scatter_accumulate_kernel<true, true>), dim3(grid2), dim3(kAccThreads), 0, stream, a, g,
                            *ta);
     } else {
         hipLaunchKernelGGL((scatter_accumulate_kernel<false, false>), dim3(grid), dim3(kAccThreads), 0, stream, a, g,
                            TableAdamArgs{});
         GRAFT_LAUNCH_CHECK();
+        if (one_phase) return;
         hipLaunchKernelGGL((scatter_accumulate_kernel<false, true>), dim3(grid2), dim3(kAccThreads), 0, stream, a, g,
                            TableAdamArgs{});
     }
