@@ -1266,8 +1266,8 @@ uint32_t InstantNerf::renderHitBatch() const
 // whole ray.  The live rays of a round are read a round later, while the next
 // one runs.  Of the 9.7 M samples of an 800 x 800 view of solid spheres 4 in 5
 // lie behind saturation.
-// With several samples per voxel (a round ends between voxels) or without an
-// output, whole rays per hit batch: compaction from the first unrendered ray,
+// With several samples per voxel (a round ends between voxels), without an
+// output or with few rays, whole rays per hit batch: compaction from the first unrendered ray,
 // one host read per hit batch; the reference makes three blocking ones.
 void InstantNerf::renderImageHit(const float3* d_rays_o, const float3* d_rays_d, uint32_t numRays, float* d_rgb_out,
                                  hipStream_t stream)
@@ -1284,7 +1284,7 @@ void InstantNerf::renderImageHit(const float3* d_rays_o, const float3* d_rays_d,
     // a render discards the prefetched rays; its whole-ray form also reuses the march store and step set 0
     b.ms[0].version = b.ms[1].version = -1;
     b.pre.valid = false;
-    if (o.samplesPerVoxel == 1 && d_rgb_out) {
+    if (o.samplesPerVoxel == 1 && d_rgb_out && graft::render_in_rounds(numRays, hitBatch)) {
         ensure_segments(b, hitBatch);
         const graft::RenderSegments& seg = b.render.seg;
         const graft::OccGrid g = occ_grid(o, d_occupancyGrid);

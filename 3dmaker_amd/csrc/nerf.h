@@ -69,6 +69,19 @@ void march_compact_stored(uint32_t R, const float3* o, const float3* d, const Oc
 constexpr int kSegmentLeast = 8, kSegmentMost = 32;
 constexpr int kSegmentRounds = kMaxHits / kSegmentLeast + 2;
 constexpr uint32_t kSegmentLast = 0x80000000u;  // in count: no sample behind this round's
+// Whether a render of R rays goes in rounds.  A round costs at least its
+// launches, about 40 us, and one more runs before the host knows that no ray
+// is left; few rays that go into a hit batch or two (20 samples a ray) are
+// faster as whole rays.
+// Whole rays against rounds in us, hit batch 2^21: 120 x 90 rays 245 / 283,
+// 160 x 120 298 / 315, 200 x 150 368 / 357, 256 x 192 497 / 435, 320 x 240
+// 859 / 526; hit batch 2^18: 120 x 90 249 / 276
+// in one hit batch and 294 / 282 in two, 160 x 120 441 / 349.
+constexpr uint32_t kSegmentRays = 24576;
+constexpr bool render_in_rounds(uint32_t R, uint32_t hit_batch)
+{
+    return R >= kSegmentRays || R > hit_batch / 20u;
+}
 struct RenderSegments {
     // per ray
     float* t;

@@ -22,6 +22,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("R,batch,cascades,bias,hidden,layers", [
     (1, 1 << 14, 1, 0.0, 64, 3),        # one ray
+    (819, 1 << 14, 1, 0.0, 64, 3),      # the most rays that go whole at this hit batch, and one more
+    (820, 1 << 14, 1, 0.0, 64, 3),
     (2047, 1 << 14, 1, 4.0, 32, 3),     # thin field: no ray saturates, many rounds
     (5000, 1 << 14, 1, -6.0, 64, 2),    # opaque field: most rays end in the first round; several chunks of rays
     (777, 1 << 12, 3, 1.0, 64, 4),      # cascades; a colour head outside the MFMA kernels' shapes
