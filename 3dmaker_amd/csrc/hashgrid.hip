@@ -4,10 +4,10 @@
 //   encode   networkFusionHashtable.cu:441-551 (encode block of the fused kernel)
 //   scatter  networkFusionBackwardHashtable.cu:783-910 (hashTableScatter_Backward)
 //
-// Thread mapping: one thread per (sample, group of 4 levels), group fastest,
-// so the per-sample row of the encoding / its gradient (4 levels x 2 features
-// = 16 B per thread) is read and written with contiguous 16-byte accesses,
-// and the level metadata comes from LDS.
+// Thread mappings: the encode deals levels to XCDs (workgroup i runs on XCD
+// i mod 8) and writes level-major encodings, from which rows are made where a
+// caller wants them; the atomic scatter has one thread per (sample, group of 4
+// levels), group fastest, and reads the gradient rows with 16-byte accesses.
 #include "hashgrid.h"
 
 #include "hash_encode.h"

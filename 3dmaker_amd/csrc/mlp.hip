@@ -1,6 +1,9 @@
 // Fully-fused TinyMLP forward/backward for gfx950 (CDNA4), fp16 MFMA with fp32
 // accumulation.
 //
+// The shapes of 16x16x32 MFMA (mlp32.hip) go there; here are the other widths,
+// the forward fused with the hash encode, and the reduction of the partials.
+//
 // Layout idea: activations travel as the B operand of v_mfma_f32_16x16x16f16
 // with samples along N and features along K.  The D layout of one 16x16 MFMA
 // (lane l holds rows 4*(l/16)..+3 of column l%16) is exactly the B layout of

@@ -8,15 +8,15 @@
 // B layout for input features 0..15, is sanitised and rounded to fp16 in
 // place; each lane adds the 4 SH coefficients of its sample it holds as
 // features 16..31.  Every value is produced by the same fp32 operations in the
-// same order as the three-launch chain, so the outputs are bitwise those of
-// that chain.  The saved buffers (density output, sigma, both heads'
+// same order as a chain of three launches on 16x16x16 MFMA; the stand-alone
+// heads sum 32 products per MFMA, so they differ in the last bits.  The saved buffers (density output, sigma, both heads'
 // activations) are the ones the backward reads; an inference caller passes
 // nulls and keeps only sigma and the colour output.
 //
 // Backward, dX part: the colour head's dX chain, the density-gradient glue
 // (compute_density_grad, otherKernels.cu:506-562) and the density head's dX
-// chain, down to dL/d(encoding) for the hash scatter; bitwise the outputs of
-// the dX-only head kernels and density_grad_kernel.  The weight gradients are
+// chain, down to dL/d(encoding) for the hash scatter; the values of the
+// dX-only head kernels (up to their order of sums) and density_grad_kernel.  The weight gradients are
 // computed apart (mlp_backward with dx = nullptr).
 #include "hashgrid.h"
 #include "mlp_device.h"
