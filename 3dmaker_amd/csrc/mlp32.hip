@@ -15,6 +15,7 @@
 // db are fp32 sums, reduced over blocks in a fixed order.
 #include "mlp.h"
 #include "mlp32.h"
+#include "mlp32_lds.h"
 
 #include "hash_encode.h"
 #include "hashgrid.h"
@@ -34,25 +35,6 @@ __device__ __forceinline__ h8 h8zero()
 {
     const _Float16 z = (_Float16)0.f;
     return h8{z, z, z, z, z, z, z, z};
-}
-
-__host__ __device__ __forceinline__ int up16(int d) { return (d + 15) & ~15; }
-__host__ __device__ __forceinline__ int up32(int d) { return (d + 31) & ~31; }
-
-// The weights in LDS: layer 0's HID rows of up32(in) halves, then the rows of
-// all other layers, HID halves each, one after another (the last layer's
-// padded to last_rows); every row is followed by 8 halves of padding
-// against bank conflicts.
-__host__ __device__ __forceinline__ int rows0_halves(int hid, int in) { return hid * (up32(in) + 8); }
-__host__ __device__ __forceinline__ int rows_halves(int hid, int in, int layers, int last_rows)
-{
-    return rows0_halves(hid, in) + ((layers - 2) * hid + last_rows) * (hid + 8);
-}
-// First LDS half of layer l's rows, and their pitch.
-template <int HID>
-__device__ __forceinline__ int row_base(int l, int in)
-{
-    return l == 0 ? 0 : rows0_halves(HID, in) + (l - 1) * HID * (HID + 8);
 }
 
 // Copies every layer's W rows into LDS, zeros outside the matrix.  Each thread
@@ -85,8 +67,8 @@ __device__ __forceinline__ void stage_rows(_Float16* sw, const _Float16* const* 
             const bool first = q < total0;
             const int row0 = (int)((unsigned)q / (unsigned)C0);
             const int e = q - total0, R = e / C;
-            const int l = first ? 0 : 1 + R / HID;
-            const int row = first ? row0 : R % HID;
+            const int l = first ? 0 : staged_layer(R, HID, layers);
+            const int row = first ? row0 : staged_row(R, HID, l);
             const int c = 8 * (first ? q - row0 * C0 : e % C);
             const int ld = first ? in : HID;
             dst[k] = first ? row * (8 * C0 + 8) + c : rows0_halves(HID, in) + R * (HID + 8) + c;
@@ -258,7 +240,7 @@ __global__ __launch_bounds__(256) void mlp32_fwd_kernel(const Fwd32Params p)
         for (int l = 0; l < p.layers - 1; l++) {
             const int KS = l == 0 ? KB0 : HB;
             const int pitch = l == 0 ? 32 * KB0 + 8 : HID + 8;
-            const _Float16* w = sw + row_base<HID>(l, p.in) + (8 * (r >> 2) + (r & 3)) * pitch + 8 * g;
+            const _Float16* w = sw + row_base(HID, p.in, l) + (8 * (r >> 2) + (r & 3)) * pitch + 8 * g;
             const float* bl = sb + l * HID + 8 * g;
             h8 Y[NT][HB];
 #pragma unroll
@@ -302,7 +284,7 @@ __global__ __launch_bounds__(256) void mlp32_fwd_kernel(const Fwd32Params p)
         const int l = p.layers - 1;
         const int pitch = HID + 8;
         const bool pairs = p.out_dim > 16;
-        const _Float16* w = sw + row_base<HID>(l, p.in) + (pairs ? 8 * (r >> 2) + (r & 3) : r) * pitch + 8 * g;
+        const _Float16* w = sw + row_base(HID, p.in, l) + (pairs ? 8 * (r >> 2) + (r & 3) : r) * pitch + 8 * g;
         const float* bl = sb + l * HID;
         const int OQ = pairs ? (p.out_dim + 31) >> 5 : 1;
         for (int q = 0; q < OQ; q++) {
@@ -562,7 +544,7 @@ __global__ __launch_bounds__(256, HB == 1 ? 4 : HB == 2 ? 2 : 1) void mlp32_bwd_
             // dX of this wave's 32 samples, rounded to fp16, masked by the input
             if (l > 0 || p.dx != nullptr) {
                 const int wp = l == 0 ? 32 * KI + 8 : HID + 8;
-                const _Float16* w = sw + row_base<HID>(l, p.in) + (8 * g + (r >> 2)) * wp + 8 * (r & 3);
+                const _Float16* w = sw + row_base(HID, p.in, l) + (8 * g + (r >> 2)) * wp + 8 * (r & 3);
                 h8 D[2][HB];
 #pragma unroll
                 for (int q = 0; q < HB; q++) {

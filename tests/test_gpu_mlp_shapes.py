@@ -86,6 +86,70 @@ def test_launchers_forward_and_backward(i, h, o, n, act, N, shift):
     assert_close(dx.cpu().numpy().reshape(N, i), rdx, what="dx")
 
 
+@pytest.mark.parametrize("grid", [False, True])
+@pytest.mark.parametrize("h,o,n,N", [(32, 64, 2, 40), (32, 128, 3, 32769), (64, 128, 4, 17), (64, 96, 2, 1)])
+def test_output_widths(h, o, n, N, grid):
+    """Outputs wider than the hidden layers: both forward launchers of each net."""
+    print(f"[mlp outputs] {h}-{o} x {n} N={N} grid={grid}", flush=True)
+    P = pkg()
+    W, B = make(32, h, o, n, 5)
+    rng = np.random.default_rng(6)
+    w16 = [w.astype(np.float16) for w in W]
+    dW16, dB = [torch.from_numpy(w).cuda() for w in w16], [torch.from_numpy(b).cuda() for b in B]
+    acts = [torch.zeros(N, 32 if l == 0 else h, dtype=torch.float16, device="cuda") for l in range(n)]
+    y, y2 = torch.zeros(N, o, device="cuda"), torch.zeros(N, o, device="cuda")
+    pa, pw, pb = pointers(acts), pointers(dW16), pointers(dB)
+    if grid:
+        T_, L, b = 1 << 12, 16, 1.3
+        table = rng.uniform(-1, 1, L * T_ * 2).astype(np.float16)
+        pos = np.zeros((N, 4), np.float32)
+        pos[:, :3] = rng.random((N, 3))
+        d_tab, d_pos = torch.from_numpy(table).cuda(), torch.from_numpy(pos).cuda()
+        opt = P.MLPGridOptions(vectorDim=4, hiddenDim=h, outputDim=o, numLayers=n, activationType=0, tableSize=T_,
+                               numLevels=L, b=b, lowestSize=16, featuresLevel=2)
+        P.launch("launchNetworkFusionHashTableGradKernel", C.byref(opt), d_tab, d_pos, pa, pw, pb, y, N, None)
+        P.launch("launchNetworkFusionHashTableKernel", C.byref(opt), d_tab, d_pos, pw, pb, y2, N, None)
+        x = orc.hash_encode(pos, table, T_, L, 16, b)
+    else:
+        x = rng.standard_normal((N, 32)).astype(np.float16)
+        acts[0].copy_(torch.from_numpy(x))
+        opt = P.MLPOption(inputDim=32, hiddenDim=h, outputDim=o, numLayers=n, activationType=0, outputActivation=0)
+        P.launch("launchNetworkFusionGradKernel", C.byref(opt), acts[0], pa, pw, pb, y, N, None)
+        P.launch("launchNetworkFusionKernel", C.byref(opt), acts[0], pw, pb, y2, N, None)
+    torch.cuda.synchronize()
+    y_ref, a_ref = orc.mlp_forward(x, flat(w16), flat(B), 32, h, o, n)
+    assert_close(y.cpu().numpy(), y_ref, what="output")
+    np.testing.assert_array_equal(y.cpu().numpy(), y2.cpu().numpy())
+    assert_close(np.stack([t.cpu().numpy() for t in acts[1:]]), a_ref, what="activations")
+
+
+def test_net_with_outputs_wider_than_its_hidden_layers():
+    """The class: forward, inference and a gradient from outside, 32 wide with 64 outputs."""
+    P = pkg()
+    N = 300
+    net = P.Net(P.MLPOption(inputDim=32, hiddenDim=32, outputDim=64, numLayers=3, activationType=0, outputActivation=0),
+                N, seed=2)
+    W, B = make(32, 32, 64, 3, 8)
+    net.load_weights(flat(W), flat(B))
+    rng = np.random.default_rng(2)
+    x, dy = rng.standard_normal((N, 32)).astype(np.float16), (rng.standard_normal((N, 64)) * 0.05).astype(np.float16)
+    out, inf = torch.zeros(N, 64, device="cuda"), torch.zeros(N, 64, device="cuda")
+    dx = torch.zeros(N, 32, dtype=torch.float16, device="cuda")
+    d_x = torch.from_numpy(x).cuda()
+    net.zero_grad()
+    net.forward(d_x, out, N)
+    net.backward(N, custom_grad=torch.from_numpy(dy).cuda(), dx_out=dx)
+    net.inference(d_x, inf, N)
+    torch.cuda.synchronize()
+    w16 = flat([w.astype(np.float16) for w in W])
+    y_ref, a_ref = orc.mlp_forward(x, w16, flat(B), 32, 32, 64, 3)
+    assert_close(out.cpu().numpy(), y_ref, what="output")
+    np.testing.assert_array_equal(out.cpu().numpy(), inf.cpu().numpy())
+    rdx = orc.mlp_backward(dy, x, a_ref, w16, 32, 32, 64, 3)[2]
+    # one fp16 rounding of a hidden unit moves a gradient by a weight times dL/dy: 2e-3 covers it
+    assert_close(dx.cpu().numpy(), rdx, what="dx")
+
+
 @pytest.mark.parametrize("N", [1, 40, 32769])
 def test_padded_ends_match_the_padded_net(N):
     """3 -> 8 inputs and 5 -> 8 outputs padded inside the kernel: activation 0, padded and caller's outputs."""
