@@ -47,7 +47,6 @@ __device__ __forceinline__ void stage_rows(_Float16* sw, const _Float16* const* 
                                            int last_rows)
 {
     constexpr int kBatch = 12;
-    constexpr int C = HID / 8;  // chunks of a row behind layer 0
     __shared__ const _Float16* sW[kMaxLayers];
     const int tid = threadIdx.x;
     if (tid < layers) sW[tid] = W[tid];
@@ -55,25 +54,17 @@ __device__ __forceinline__ void stage_rows(_Float16* sw, const _Float16* const* 
     uintptr_t low = 0;
     for (int l = 0; l < layers; l++) low |= reinterpret_cast<uintptr_t>(sW[l]);
     const bool vec = __builtin_amdgcn_readfirstlane((int)(low & 15u)) == 0;
-    const int C0 = up32(in) >> 3, total0 = HID * C0;
-    const int total = total0 + ((layers - 2) * HID + last_rows) * C;
+    const int total = staged_chunks(HID, in, layers, last_rows);
     for (int base = 0; base < total; base += kBatch * (int)blockDim.x) {
         h8 v[kBatch];
         int dst[kBatch];
         bool ok[kBatch];
 #pragma unroll
         for (int k = 0; k < kBatch; k++) {
-            const int q = min(base + k * (int)blockDim.x + tid, total - 1);
-            const bool first = q < total0;
-            const int row0 = (int)((unsigned)q / (unsigned)C0);
-            const int e = q - total0, R = e / C;
-            const int l = first ? 0 : staged_layer(R, HID, layers);
-            const int row = first ? row0 : staged_row(R, HID, l);
-            const int c = 8 * (first ? q - row0 * C0 : e % C);
-            const int ld = first ? in : HID;
-            dst[k] = first ? row * (8 * C0 + 8) + c : rows0_halves(HID, in) + R * (HID + 8) + c;
-            ok[k] = c < ld && (l < layers - 1 || row < out);
-            const _Float16* src = sW[l] + (ok[k] ? row * ld + c : 0);
+            const Staged c = staged_chunk(min(base + k * (int)blockDim.x + tid, total - 1), HID, in, out, layers);
+            dst[k] = c.dst;
+            ok[k] = c.ok;
+            const _Float16* src = sW[c.layer] + (c.ok ? c.at : 0);
             if (vec) {
                 v[k] = *reinterpret_cast<const h8*>(src);
             } else {
@@ -146,7 +137,7 @@ __global__ __launch_bounds__(256) void mlp32_fwd_kernel(const Fwd32Params p)
     _Float16* sw = reinterpret_cast<_Float16*>(smem);
     float* sb = reinterpret_cast<float*>(smem + p.bias_base);
     // the first two biases of a thread are on their way while the weights are staged
-    const int tid = threadIdx.x, nb = (p.layers - 1) * HID + up16(p.out_dim);
+    const int tid = threadIdx.x, nb = fwd32_biases(HID, p.out_dim, p.layers);
     auto bias = [&](int e) {
         const int l = min(e / HID, p.layers - 1), i = e - l * HID;
         const bool ok = e < nb && i < (l == p.layers - 1 ? p.out_dim : HID);
@@ -154,7 +145,7 @@ __global__ __launch_bounds__(256) void mlp32_fwd_kernel(const Fwd32Params p)
         return ok ? v : 0.f;
     };
     const float b0 = bias(tid), b1 = bias(tid + 256);
-    stage_rows<HID>(sw, p.W, p.in, p.out_dim, p.layers, up16(p.out_dim));
+    stage_rows<HID>(sw, p.W, p.in, p.out_dim, p.layers, fwd32_last_rows(p.out_dim));
     if (tid < nb) sb[tid] = b0;
     if (tid + 256 < nb) sb[tid + 256] = b1;
     for (int e = tid + 512; e < nb; e += 256) sb[e] = bias(e);
@@ -240,7 +231,7 @@ __global__ __launch_bounds__(256) void mlp32_fwd_kernel(const Fwd32Params p)
         for (int l = 0; l < p.layers - 1; l++) {
             const int KS = l == 0 ? KB0 : HB;
             const int pitch = l == 0 ? 32 * KB0 + 8 : HID + 8;
-            const _Float16* w = sw + row_base(HID, p.in, l) + (8 * (r >> 2) + (r & 3)) * pitch + 8 * g;
+            const _Float16* w = sw + row_base(HID, p.in, l) + fwd32_lane_row(true, r) * pitch + 8 * g;
             const float* bl = sb + l * HID + 8 * g;
             h8 Y[NT][HB];
 #pragma unroll
@@ -283,15 +274,15 @@ __global__ __launch_bounds__(256) void mlp32_fwd_kernel(const Fwd32Params p)
         // last layer: blocks of 16 outputs when there are at most 16, else pairs
         const int l = p.layers - 1;
         const int pitch = HID + 8;
-        const bool pairs = p.out_dim > 16;
-        const _Float16* w = sw + row_base(HID, p.in, l) + (pairs ? 8 * (r >> 2) + (r & 3) : r) * pitch + 8 * g;
+        const bool pairs = fwd32_pairs(p.out_dim);
+        const _Float16* w = sw + row_base(HID, p.in, l) + fwd32_lane_row(pairs, r) * pitch + 8 * g;
         const float* bl = sb + l * HID;
-        const int OQ = pairs ? (p.out_dim + 31) >> 5 : 1;
+        const int OQ = fwd32_last_steps(p.out_dim);
         for (int q = 0; q < OQ; q++) {
 #pragma unroll
             for (int m = 0; m < 2; m++) {
                 if (m == 1 && !pairs) continue;
-                const int col = pairs ? 32 * q + 8 * g + 4 * m : 4 * g;
+                const int col = fwd32_lane_col(pairs, q, m, g);
                 f4 acc[NT];
 #pragma unroll
                 for (int t = 0; t < NT; t++) acc[t] = *reinterpret_cast<const f4*>(bl + col);
@@ -370,8 +361,6 @@ void pick_fwd32(const Fwd32Params& p, int mode, bool save, int act, int lds, int
     }
 }
 
-int fwd32_bias_base(const MlpShape& s) { return (rows_halves(s.hid, s.in, s.layers, up16(s.out)) * 2 + 15) & ~15; }
-int fwd32_lds(const MlpShape& s) { return fwd32_bias_base(s) + 4 * ((s.layers - 1) * s.hid + up16(s.out)); }
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // ---------------------------------------------------------------------------
@@ -670,7 +659,7 @@ bool mlp32_forward_supported(const MlpShape& s)
 {
     if (s.layers < 2 || (s.hid != 32 && s.hid != 64 && s.hid != 128)) return false;
     if (s.in % 8 || s.in > 128 || s.out % 4 || s.out > 128) return false;
-    return fwd32_lds(s) + kStaticLds <= max_lds_per_block();
+    return fwd32_lds(s.in, s.hid, s.out, s.layers) + kStaticLds <= max_lds_per_block();
 }
 
 void mlp32_forward(const MlpShape& s, const FwdInput& in, const __half* const* W, const float* const* B,
@@ -684,8 +673,8 @@ void mlp32_forward(const MlpShape& s, const FwdInput& in, const __half* const* W
     p.in = s.in;
     p.out_dim = s.out;
     p.layers = s.layers;
-    p.bias_base = fwd32_bias_base(s);
-    const int lds = fwd32_lds(s);
+    p.bias_base = fwd32_bias_base(s.in, s.hid, s.out, s.layers);
+    const int lds = fwd32_lds(s.in, s.hid, s.out, s.layers);
     p.x_dim = in.x_dim > 0 ? in.x_dim : s.in;
     p.save_x0 = in.save_x0 ? 1 : 0;
     p.user_dim = in.user_dim > 0 ? in.user_dim : s.out;

@@ -87,9 +87,11 @@ def test_launchers_forward_and_backward(i, h, o, n, act, N, shift):
 
 
 @pytest.mark.parametrize("grid", [False, True])
-@pytest.mark.parametrize("h,o,n,N", [(32, 64, 2, 40), (32, 128, 3, 32769), (64, 128, 4, 17), (64, 96, 2, 1)])
+@pytest.mark.parametrize("h,o,n,N", [(32, 64, 2, 40), (32, 128, 3, 32769), (64, 128, 4, 17), (64, 96, 2, 1),
+                                     (32, 36, 2, 40), (64, 48, 2, 32769), (128, 80, 3, 33), (64, 112, 4, 17),
+                                     (32, 100, 3, 257), (128, 112, 2, 1), (64, 40, 3, 100)])
 def test_output_widths(h, o, n, N, grid):
-    """Outputs wider than the hidden layers: both forward launchers of each net."""
+    """Outputs wider than the hidden layers, and widths whose last pair of 16-row blocks is one of padding: both forward launchers of each net."""
     print(f"[mlp outputs] {h}-{o} x {n} N={N} grid={grid}", flush=True)
     P = pkg()
     W, B = make(32, h, o, n, 5)
