@@ -158,7 +158,7 @@ void launchNetworkFusionHashTableKernel(MLPGridOptions* opt, half* d_hashtable, 
         in.pos_stride = 4;
         in.table = d_hashtable;
         in.meta = &m;
-        in.scratch = &graft::stream_encode_scratch(stream);
+        in.scratch = &graft::launcher_encode_scratch();
         graft::mlp_forward(shape(opt), in, W, B, nullptr, d_outputs, batchSize, OUT_ACT_NONE, stream);
     });
 }
@@ -174,7 +174,7 @@ void launchNetworkFusionHashTableGradKernel(MLPGridOptions* opt, half* d_hashtab
         in.pos_stride = 4;
         in.table = d_hashtable;
         in.meta = &m;
-        in.scratch = &graft::stream_encode_scratch(stream);
+        in.scratch = &graft::launcher_encode_scratch();
         graft::mlp_forward(shape(opt), in, W, B, acts, d_outputs, batchSize, OUT_ACT_NONE, stream);
     });
 }
@@ -247,7 +247,7 @@ void launchHashEncodeKernel(MLPGridOptions* opt, half* d_hashtable, const float*
     guarded("launchHashEncodeKernel", [&] {
         const graft::GridMeta m = meta(opt);
         graft::hash_encode(m, d_hashtable, d_inputs, inputStride, d_enc_out, batchSize, stream, nullptr,
-                           &graft::stream_encode_scratch(stream));
+                           &graft::launcher_encode_scratch());
     });
 }
 

@@ -95,12 +95,10 @@ public:
     Workspace(const Workspace&) = delete;
     Workspace& operator=(const Workspace&) = delete;
     void* get(size_t bytes);
-    // At least `bytes` for work on stream s, or nullptr (what is held stays)
-    // when the stream is being captured (a graph would keep an address that a
-    // later call may free), is hipStreamPerThread or the memory cannot be had:
+    // As get(), but nullptr (what is held stays) when the memory cannot be had:
     // for callers that have another way.  mutex() is theirs to hold while they
     // enqueue what uses it.
-    void* try_get(size_t bytes, hipStream_t s);
+    void* try_get(size_t bytes);
     std::mutex& mutex() { return mu_; }
     size_t size() const { return bytes_; }
 
@@ -113,19 +111,33 @@ private:
 // The workspace of (current device, stream), for callers without an owner of
 // their own (the extern "C" launchers); kept until the process ends.
 Workspace& stream_workspace(hipStream_t s);
-// One Workspace per (device, stream) a caller works on: calls of several
-// threads and streams each find their stream's, and all go with the owner.
+
+// One Workspace per (device, stream) that its callers work on, for callers that
+// have another way: calls of several threads and streams each find their
+// stream's.  It holds at most kMost of them; a stream beyond those gets one
+// when another has not asked for its own in the last kIdle calls (that one is
+// given back, so that streams that are gone do not keep theirs).  A workspace
+// stays while a call holds it.
 class StreamScratch {
 public:
-    Workspace& of(hipStream_t s);
+    static constexpr size_t kMost = 4;
+    static constexpr uint64_t kIdle = 64;
+    // nullptr also for a stream under capture (a graph would keep an address
+    // that a later call may free) and for hipStreamPerThread.
+    std::shared_ptr<Workspace> of(hipStream_t s);
 
 private:
+    struct Held {
+        std::shared_ptr<Workspace> ws;
+        uint64_t used = 0;
+    };
     std::mutex mu_;
-    std::map<std::pair<int, hipStream_t>, std::unique_ptr<Workspace>> ws_;
+    uint64_t calls_ = 0;
+    std::map<std::pair<int, hipStream_t>, Held> held_;
 };
 
 // That of the extern "C" launchers for level-major encodings.
-Workspace& stream_encode_scratch(hipStream_t s);
+StreamScratch& launcher_encode_scratch();
 
 int num_cus();
 

@@ -8,10 +8,11 @@ namespace graft {
 // enc [N x 2L] fp16 from positions [N x pos_stride] (x, y, z, ...).
 // d_n (nullable): device-side sample count (<= N), as for the MLP kernels.
 // scratch (nullable): room for level-major encodings, with which large batches
-// are faster.
+// are faster, kEncodePiece samples at a time.
+constexpr int kEncodePiece = 1 << 20;
 void hash_encode(const GridMeta& m, const __half* table, const float* pos, int pos_stride,
                  __half* enc, int N, hipStream_t stream, const uint32_t* d_n = nullptr,
-                 Workspace* scratch = nullptr);
+                 StreamScratch* scratch = nullptr);
 
 // The same encodings level-major: level l of sample n at enc[(l * plane + n) * 2],
 // its two features adjacent (plane >= N).  scattered: the positions come in no

@@ -260,24 +260,31 @@ void launch_encode(const GridMeta& m, const __half* table, const float* pos, int
 }  // namespace
 
 // Row-major output costs the encode a partial line per level and sample; from
-// kRowsFromPlanar samples on, level-major encodings in `scratch` and a pass
-// that turns them into rows are the faster way.  The two launches are
-// enqueued under the scratch's lock, so that calls of several threads on one
-// stream do not come between each other's.
+// kRowsFromPlanar samples on, level-major encodings in the stream's scratch and
+// a pass that turns them into rows are the faster way, kEncodePiece samples at
+// a time so that what is kept has a bound.  The launches are enqueued under the
+// scratch's lock, so that calls of several threads on one stream do not come
+// between each other's.
 void hash_encode(const GridMeta& m, const __half* table, const float* pos, int pos_stride,
-                 __half* enc, int N, hipStream_t stream, const uint32_t* d_n, Workspace* scratch)
+                 __half* enc, int N, hipStream_t stream, const uint32_t* d_n, StreamScratch* scratch)
 {
     if (N <= 0) return;
     if (pos_stride < 3) throw std::runtime_error("hash encode: position stride must be >= 3");
     constexpr int kRowsFromPlanar = 1 << 15;
-    if (scratch && !d_n && N >= kRowsFromPlanar) {
-        std::lock_guard<std::mutex> lk(scratch->mutex());
-        if (void* planar = scratch->try_get((size_t)N * m.numLevels * 2 * sizeof(__half), stream)) {
-            launch_encode<true, true>(m, table, pos, pos_stride, static_cast<__half*>(planar), N, N, stream, nullptr);
-            hipLaunchKernelGGL(encode_rows_kernel, dim3(std::min((N + 63) / 64, 1 << 20)), dim3(256), 0, stream,
-                               static_cast<const _Float16*>(planar), N, m.numLevels, N,
-                               reinterpret_cast<_Float16*>(enc));
-            GRAFT_LAUNCH_CHECK();
+    const std::shared_ptr<Workspace> ws = scratch && !d_n && N >= kRowsFromPlanar ? scratch->of(stream) : nullptr;
+    if (ws) {
+        const int D = 2 * m.numLevels, piece = std::min(N, kEncodePiece);
+        std::lock_guard<std::mutex> lk(ws->mutex());
+        if (void* planar = ws->try_get((size_t)piece * D * sizeof(__half))) {
+            for (int n0 = 0; n0 < N; n0 += piece) {
+                const int n = std::min(piece, N - n0);
+                launch_encode<true, true>(m, table, pos + (size_t)n0 * pos_stride, pos_stride,
+                                          static_cast<__half*>(planar), piece, n, stream, nullptr);
+                hipLaunchKernelGGL(encode_rows_kernel, dim3((n + 63) / 64), dim3(256), 0, stream,
+                                   static_cast<const _Float16*>(planar), piece, m.numLevels, n,
+                                   reinterpret_cast<_Float16*>(enc) + (size_t)n0 * D);
+                GRAFT_LAUNCH_CHECK();
+            }
             return;
         }
     }
@@ -355,14 +362,8 @@ void* Workspace::get(size_t bytes)
     return p_;
 }
 
-void* Workspace::try_get(size_t bytes, hipStream_t s)
+void* Workspace::try_get(size_t bytes)
 {
-    // hipStreamPerThread names another stream in every thread
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (s == hipStreamPerThread || hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
     if (bytes <= bytes_) return p_;
     void* p = nullptr;
     if (hipMalloc(&p, bytes) != hipSuccess) {
@@ -375,20 +376,39 @@ void* Workspace::try_get(size_t bytes, hipStream_t s)
     return p_;
 }
 
-Workspace& StreamScratch::of(hipStream_t s)
+std::shared_ptr<Workspace> StreamScratch::of(hipStream_t s)
 {
+    // hipStreamPerThread names another stream in every thread
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (s == hipStreamPerThread || hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
     int dev = 0;
     GRAFT_HIP_CHECK(hipGetDevice(&dev));
+    std::shared_ptr<Workspace> given_back;  // freed behind the lock
     std::lock_guard<std::mutex> lk(mu_);
-    auto& w = ws_[{dev, s}];
-    if (!w) w.reset(new Workspace());
-    return *w;
+    calls_++;
+    auto at = held_.find({dev, s});
+    if (at == held_.end()) {
+        if (held_.size() >= kMost) {
+            auto old = held_.begin();
+            for (auto i = held_.begin(); i != held_.end(); ++i)
+                if (i->second.used < old->second.used) old = i;
+            if (calls_ - old->second.used <= kIdle) return nullptr;
+            given_back = std::move(old->second.ws);
+            held_.erase(old);
+        }
+        at = held_.emplace(std::make_pair(dev, s), Held{std::make_shared<Workspace>(), 0}).first;
+    }
+    at->second.used = calls_;
+    return at->second.ws;
 }
 
-Workspace& stream_encode_scratch(hipStream_t s)
+StreamScratch& launcher_encode_scratch()
 {
     static StreamScratch* all = new StreamScratch();  // outlives static destructors
-    return all->of(s);
+    return *all;
 }
 
 Workspace& stream_workspace(hipStream_t s)

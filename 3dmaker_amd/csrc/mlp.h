@@ -32,7 +32,7 @@ struct FwdInput {
     int x_dim = 0;
     float* user = nullptr;
     int user_dim = 0;
-    Workspace* scratch = nullptr;
+    StreamScratch* scratch = nullptr;
 };
 bool mlp_forward_wide(const MlpShape& s);
 

@@ -6,10 +6,8 @@
 
 namespace graft {
 
-// Samples from which the hash-grid forward encodes in a launch of its own, and
-// the samples that share one piece of its scratch in inference.
+// Samples from which the hash-grid forward encodes in a launch of its own.
 constexpr int kPlanarFrom = 1 << 15;
-constexpr int kPlanarPiece = 1 << 20;
 
 bool mlp32_forward_supported(const MlpShape& s);
 void mlp32_forward(const MlpShape& s, const FwdInput& in, const __half* const* W, const float* const* B,

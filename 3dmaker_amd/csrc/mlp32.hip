@@ -116,6 +116,7 @@ struct Fwd32Params {
     float* user;               // nullable [N x user_dim]: the first user_dim outputs again
     const uint32_t* d_n;
     int N, in, out_dim, layers, pos_stride, plane, x_dim, user_dim;
+    int row0;                  // the batch's first row in acts
     int save_x0, vec_x, vec_out, vec_user;
     int L, T, dense_start;
     int bias_base;  // bytes into LDS; layer l's biases HID floats apart
@@ -157,7 +158,7 @@ __global__ __launch_bounds__(256) void mlp32_fwd_kernel(const Fwd32Params p)
     const int KB0 = (p.in + 31) >> 5;
     constexpr int XB = 4;  // 32-feature blocks of the widest input
     _Float16* act0 = nullptr;
-    if constexpr (SAVE) act0 = p.acts[0];
+    if constexpr (SAVE) act0 = p.acts[0] + (size_t)p.row0 * p.in;
 
     auto load = [&](int u, h8 (&X)[NT][XB]) {
 #pragma unroll
@@ -260,7 +261,7 @@ __global__ __launch_bounds__(256) void mlp32_fwd_kernel(const Fwd32Params p)
                     }
             }
             _Float16* act = nullptr;
-            if constexpr (SAVE) act = p.acts[l + 1];
+            if constexpr (SAVE) act = p.acts[l + 1] + (size_t)p.row0 * HID;
 #pragma unroll
             for (int t = 0; t < NT; t++) {
                 const int n = (u * NT + t) * 16 + r;
@@ -682,6 +683,7 @@ void mlp32_forward(const MlpShape& s, const FwdInput& in, const __half* const* W
     const int act = in.table ? 0 : out_act;  // the hash-grid net has no output activation
     auto run = [&](int mode, int n0, int n) {
         p.N = n;
+        p.row0 = n0;
         const int xs = p.x_dim;
         if (in.x) p.x = reinterpret_cast<const _Float16*>(in.x) + (size_t)n0 * xs;
         p.vec_x = xs == s.in && aligned16(p.x);
@@ -713,12 +715,12 @@ void mlp32_forward(const MlpShape& s, const FwdInput& in, const __half* const* W
     // Encodings first, level-major into scratch, then the net on them: the
     // encode then works on one table at a time per XCD.  One launch for
     // everything below kPlanarFrom samples, where its shorter chain wins, and
-    // where no scratch is to be had.  Saved activations hold one batch, so
-    // only inference is cut into pieces that bound the scratch.
-    if (in.scratch && !d_n && N >= kPlanarFrom) {
-        const int piece = save ? N : std::min(N, kPlanarPiece);
-        std::lock_guard<std::mutex> lk(in.scratch->mutex());
-        if (void* enc = in.scratch->try_get((size_t)piece * m.numLevels * 2 * sizeof(__half), stream)) {
+    // where no scratch is to be had.  Pieces of kEncodePiece bound the scratch.
+    const std::shared_ptr<Workspace> ws = in.scratch && !d_n && N >= kPlanarFrom ? in.scratch->of(stream) : nullptr;
+    if (ws) {
+        const int piece = std::min(N, kEncodePiece);
+        std::lock_guard<std::mutex> lk(ws->mutex());
+        if (void* enc = ws->try_get((size_t)piece * m.numLevels * 2 * sizeof(__half))) {
             p.enc = static_cast<const _Float16*>(enc);
             p.plane = piece;
             for (int n0 = 0; n0 < N; n0 += piece) {

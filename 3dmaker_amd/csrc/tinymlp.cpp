@@ -707,7 +707,7 @@ void TinyMLPHashGrid::forward(const float* d_unpadded_inputs, float* d_outputs, 
     in.pos_stride = 4;
     in.table = d_fwd_hashtable;
     in.meta = &META;
-    in.scratch = &ENCODE.of(stream);
+    in.scratch = &ENCODE;
     const bool wide = graft::mlp_forward_wide(shape_of(mlp_opt));
     in.user = d_outputs;  // the wide kernel stores the caller's outputs too
     in.user_dim = user_opt.outputDim;
@@ -741,7 +741,7 @@ void TinyMLPHashGrid::inference(const float* d_unpadded_inputs, float* d_outputs
     in.pos_stride = user_opt.vectorDim;
     in.table = d_fwd_hashtable;
     in.meta = &META;
-    in.scratch = &ENCODE.of(stream);
+    in.scratch = &ENCODE;
     if (user_opt.outputDim == hw_opt.outputDim) {
         if (d_outputs)
             graft::mlp_forward(shape_of(mlp_opt), in, d_fwd_weights, d_master_biases, nullptr, d_outputs, batchSize,
