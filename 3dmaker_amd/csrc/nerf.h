@@ -73,10 +73,11 @@ constexpr uint32_t kSegmentLast = 0x80000000u;  // in count: no sample behind th
 // launches, about 40 us, and one more runs before the host knows that no ray
 // is left; few rays that go into a hit batch or two (20 samples a ray) are
 // faster as whole rays.
-// Whole rays against rounds in us, hit batch 2^21: 120 x 90 rays 245 / 283,
-// 160 x 120 298 / 315, 200 x 150 368 / 357, 256 x 192 497 / 435, 320 x 240
-// 859 / 526; hit batch 2^18: 120 x 90 249 / 276
-// in one hit batch and 294 / 282 in two, 160 x 120 441 / 349.
+// Whole rays against rounds in us, hit batch 2^21: 120 x 90 rays 218 / 256,
+// 160 x 120 264 / 289, 180 x 135 293 / 310 (292 / 289 in another scene), 200 x
+// 150 324 / 330 (319 / 306), 256 x 192 431 / 402, 320 x 240 737 / 484; hit batch
+// 2^18: 100 x 75 198 / 246, 120 x 90 279 / 259 (two hit batches), 140 x 105
+// 301 / 312, 160 x 120 388 / 343, 201 x 151 512 / 368.
 constexpr uint32_t kSegmentRays = 24576;
 constexpr bool render_in_rounds(uint32_t R, uint32_t hit_batch)
 {

@@ -100,7 +100,7 @@ def test_many_streams_keep_few_workspaces():
 def test_forward_with_saved_activations_in_pieces():
     """The gradient launcher over several pieces: saved encodings, hidden activations and outputs."""
     P = pkg()
-    N, hid, out = PIECE + 777, 32, 16
+    N, hid, out = 3 * PIECE + 777, 32, 16
     tab, pos = table(), positions(N, 4)
     g = torch.Generator("cuda").manual_seed(5)
     dims = [(hid, 2 * L), (hid, hid), (out, hid)]

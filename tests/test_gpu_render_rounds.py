@@ -82,3 +82,40 @@ def test_render_matches_whole_rays(R, batch, cascades, bias, hidden, layers):
     if cascades == 1 and R > 1:
         assert cnt.max() > 17  # more than one round
     nerf.close()
+
+
+@pytest.mark.parametrize("hidden,layers", [(32, 3), (64, 2), (64, 4)])   # the last one outside the MFMA heads
+def test_a_ray_has_one_colour_however_rays_are_grouped(hidden, layers):
+    """The same rays in one call (rounds), in calls small enough to go whole, alone, and with another hit batch: the
+    same bits."""
+    P = pkg()
+    res, mips, T_, R, batch = 64, 4, 1 << 14, 3000, 1 << 14
+    small = batch // 20                  # the most rays that go whole
+    o = P.Nerf.default_options()
+    o.gridResolution[:] = [res] * 3
+    o.aabbMin[:], o.aabbMax[:] = [-1.5] * 3, [1.5] * 3
+    o.levelsMipmap, o.numCascades, o.samplesPerVoxel = mips, 1, 1
+    o.hashTableSize, o.growthFactor = T_, 1.447
+    o.colorHiddenDim, o.colorNumLayers = hidden, layers
+    o.batchSize, o.rayChunkSize, o.renderBatchSize = batch, 512, 1 << 16
+    nerf = P.Nerf(o)
+    rng = np.random.default_rng(3)
+    nerf.density.load_hashgrid(rng.normal(0, 0.5, 16 * T_ * 2).astype(np.float32))
+    nerf.set_occupancy(scenes.pack_grid([rng.random((res, res, res)) < 0.3], mips))
+    ro, rd = scenes.rays_c4(R, n_cams=8, seed=6)
+    d_o, d_d = torch.from_numpy(ro).cuda(), torch.from_numpy(rd).cuda()
+
+    def render(cuts):
+        rgb = torch.full((R, 3), -1.0, device="cuda")
+        for a, b in zip(cuts[:-1], cuts[1:]):
+            nerf.render(d_o[a:b], d_d[a:b], b - a, rgb[a:b])
+        torch.cuda.synchronize()
+        return rgb.cpu().numpy()
+
+    whole = render([0, R])
+    assert len(np.unique(whole[:, 0])) > R // 2   # colours, not the background
+    np.testing.assert_array_equal(render(list(range(0, R, small)) + [R]), whole)
+    np.testing.assert_array_equal(render([0, 1, 2, 17, small + 17, R]), whole)
+    nerf.set_memory_mode(True)                    # a hit batch of 2^16: R <= 2^16 / 20 goes whole
+    np.testing.assert_array_equal(render([0, R]), whole)
+    nerf.close()
