@@ -707,20 +707,8 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
             graft::render_grad(ca, ga, d_rays, R, stream);
         });
         // The hash scatter waits only for dL/d(encoding): the main stream runs
-        // the dX chain of both heads (dX-only kernels for the NeRF shapes) and
-        // the side stream the weight gradients and MLP Adam beside the scatter.
-        graft::NerfBwdDxArgs bx;
-        bx.cshape = cshape;
-        bx.dshape = dshape;
-        bx.color_dy = cb.dloss;
-        bx.cacts = cb.activations;
-        bx.cW = cb.fwd_weights;
-        bx.dsigma = b.dsigma;
-        bx.dacts = db.activations;
-        bx.dW = db.fwd_weights;
-        bx.color_dx = b.color_dx;
-        bx.density_dy = db.dloss;
-        bx.denc = db.dx_out;
+        // the dX chain of both heads and the side stream their weight gradients
+        // and the MLP Adam beside the scatter.
         graft::NerfHeadsBwd hb;
         hb.packed = b.heads_packed;
         hb.color_hidden = cshape.hid;
@@ -736,27 +724,9 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
         hb.color_dx = m_keepColorDx ? b.color_dx : nullptr;  // read by nothing in the step
         hb.tile_live = b.tile_live;
         const bool heads = b.heads_packed != nullptr;
-        const bool fused_dx = !heads && graft::nerf_backward_dx(bx, 0, stream);  // shape check only (N = 0)
-        const bool dx_only = !heads && graft::mlp_has_dx_kernel(cshape) && graft::mlp_has_dx_kernel(dshape);
         if (heads) {
             // recomputed activations: colour dX chain, glue, density dX chain
             stage("backwardDx", [&] { graft::nerf_heads_dx(hb, (int)Bn, stream, d_hits); });
-        } else if (fused_dx || dx_only) {
-            if (fused_dx) {
-                // colour dX chain, density-gradient glue, density dX chain: one launch
-                stage("backwardDx", [&] { graft::nerf_backward_dx(bx, (int)Bn, stream, d_hits); });
-            } else {
-                stage("colorDx", [&] {
-                    graft::mlp_backward_dx(cshape, cb.dloss, cb.activations, cb.fwd_weights, b.color_dx, (int)Bn,
-                                           stream, d_hits);
-                });
-                stage("densityGrad",
-                      [&] { graft::density_grad(d_hits, Bn, b.dsigma, b.color_dx, db.dloss, stream); });
-                stage("densityDx", [&] {
-                    graft::mlp_backward_dx(dshape, db.dloss, db.activations, db.fwd_weights, db.dx_out, (int)Bn,
-                                           stream, d_hits);
-                });
-            }
         } else {
             stage("colorBwd", [&] {
                 graft::mlp_backward(cshape, cb.dloss, cb.activations, cb.fwd_weights, cb.w_grad, cb.b_grad,
@@ -846,17 +816,6 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
             stage_on(b.side, "headsBwd", [&] {
                 graft::nerf_heads_dw(hb, graft::NerfHeadsGrads{db.w_grad, db.b_grad, cb.w_grad, cb.b_grad}, (int)Bn,
                                      b.side, d_hits, static_cast<graft::Workspace*>(db.workspace));
-            });
-        } else if (fused_dx || dx_only) {
-            stage_on(b.side, "colorBwd", [&] {
-                graft::mlp_backward(cshape, cb.dloss, cb.activations, cb.fwd_weights, cb.w_grad, cb.b_grad, nullptr,
-                                    (int)Bn, b.side, d_hits, /*accumulate=*/false,
-                                    static_cast<graft::Workspace*>(cb.workspace));
-            });
-            stage_on(b.side, "densityBwd", [&] {
-                graft::mlp_backward(dshape, db.dloss, db.activations, db.fwd_weights, db.w_grad, db.b_grad, nullptr,
-                                    (int)Bn, b.side, d_hits, /*accumulate=*/false,
-                                    static_cast<graft::Workspace*>(db.workspace));
             });
         }
         // Adam: MLP layers of both heads on the side stream, the hash table on

@@ -53,22 +53,14 @@ void mlp_backward(const MlpShape& s, const __half* dy, const __half* const* acts
                   hipStream_t stream, const uint32_t* d_n = nullptr, bool accumulate = true,
                   Workspace* ws = nullptr);
 
-// dx = dL/dx alone, with the rounding points of mlp_backward, for the NeRF head shapes
-// (32-64-16, 2 layers; 32-64-8, 3 layers); returns false for other shapes.
-// mlp_backward(..., dx = nullptr) then yields the weight gradients.
-bool mlp_backward_dx(const MlpShape& s, const __half* dy, const __half* const* acts, const __half* const* W,
-                     __half* dx, int N, hipStream_t stream, const uint32_t* d_n = nullptr);
-bool mlp_has_dx_kernel(const MlpShape& s);
-
 // Fixed-order sum of nparts block partials ws [nparts][P] of one net's
 // gradients (W of every layer row-major [out][in], then b of every layer)
 // into dW / dB (device arrays of per-layer pointers), added when accumulate.
 void mlp_grad_reduce(const MlpShape& s, const float* ws, int nparts, float* const* dW, float* const* dB,
                      bool accumulate, hipStream_t stream);
 
-// The forward of a NeRF step (hash encode + density head, SH gather, colour
-// head) in one launch: mlp_forward(density), sh_gather,
-// mlp_forward(colour).  dacts / density_out / cacts / color_in may be null
+// The forward of a NeRF batch: hash encode, then mlp_forward(density),
+// sh_gather and mlp_forward(colour) in one launch.  dacts / density_out / cacts / color_in may be null
 // (inference); sigma and color_out are always written.
 struct NerfFwdArgs {
     MlpShape dshape;                 // density head, out == 16
@@ -92,39 +84,19 @@ struct NerfFwdArgs {
     __half* const* cacts = nullptr;  // device array; entries 1.. receive the hidden activations
     __half* color_in = nullptr;      // [N x 32] logits | SH (the colour head's activation 0)
     float* color_out = nullptr;      // [N x cshape.out]
-    // Nullable: [L][enc_plane] feature pairs (enc_plane >= N).  When set, the
-    // encode runs first as its own launch (hash_encode_planar, each XCD's L2
-    // holding only its levels' tables) and the network kernel reads it.
+    // [L][enc_plane] feature pairs (enc_plane >= N): the encode runs first, as
+    // its own launch (hash_encode_planar, each XCD's L2 holding only its levels'
+    // tables), and the network kernel reads it.
     __half* enc_scratch = nullptr;
     int enc_plane = 0;
     bool enc_ready = false;  // enc_scratch already holds these positions' encodings: no encode launch
-    // Nullable: a buffer of nerf_heads_packed_bytes().  With it, the planar
-    // encodings and the head shapes nerf_heads_supported() accepts, and no
-    // activations asked for (dacts, cacts null), the heads run as the
+    // Nullable: a buffer of nerf_heads_packed_bytes().  With it, the head
+    // shapes nerf_heads_supported() accepts, and no activations asked for (dacts, cacts null), the heads run as the
     // 16x16x32 MFMA kernels of nerf_heads.hip after packing the weights into
     // this buffer (heads_prepacked: the caller packed the current weights).
     void* heads_packed = nullptr;
     bool heads_prepacked = false;
 };
 void nerf_forward(const NerfFwdArgs& a, int N, hipStream_t stream, const uint32_t* d_n = nullptr);
-
-// The dX part of a NeRF step's backward in one launch: colour dL/dinput,
-// density dL/dy (colour dL/dinput[0..15] + d sigma on the logit, clamped) and
-// dL/d(encoding): mlp_backward_dx(colour), density_grad,
-// mlp_backward_dx(density).  Only for the head shapes 32-64-64-8 and
-// 32-64-16; returns false for others.
-struct NerfBwdDxArgs {
-    MlpShape cshape, dshape;
-    const __half* color_dy = nullptr;       // [N x 8]
-    const __half* const* cacts = nullptr;
-    const __half* const* cW = nullptr;
-    const float* dsigma = nullptr;          // [N]
-    const __half* const* dacts = nullptr;
-    const __half* const* dW = nullptr;
-    __half* color_dx = nullptr;             // [N x 32]
-    __half* density_dy = nullptr;           // [N x 16]
-    __half* denc = nullptr;                 // [N x 32]
-};
-bool nerf_backward_dx(const NerfBwdDxArgs& a, int N, hipStream_t stream, const uint32_t* d_n = nullptr);
 
 }  // namespace graft

@@ -341,38 +341,6 @@ __global__ __launch_bounds__(256) void mlp_bwd_kernel(const BwdParams p)
     }
 }
 
-// dL/dx alone (no dW/db) for the NeRF head shapes.  A caller that needs dx first (the hash scatter waits for it) runs this,
-// and the weight gradients later with mlp_backward(dx = nullptr), which
-// recomputes the chain beside other work.
-template <int IN, int HID, int OUT, int LAYERS>
-__global__ __launch_bounds__(256) void mlp_bwd_dx_kernel(const BwdParams p)
-{
-    using S = HeadShape<IN, HID, OUT, LAYERS>;
-    extern __shared__ __align__(16) unsigned char smem[];
-    _Float16* sfrag = reinterpret_cast<_Float16*>(smem);
-    stage_fragments<true>(sfrag, p.W, IN, HID, OUT, LAYERS);
-
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, g = lane >> 4, r = lane & 15;
-    const int N = p.d_n ? min((int)*p.d_n, p.N) : p.N;
-    const int ntiles = (N + 15) >> 4;
-    for (int tile = blockIdx.x * 4 + wave; tile < ntiles; tile += gridDim.x * 4) {
-        const int n = tile * 16 + r;
-        const bool valid = n < N;
-        h4 G[4];
-#pragma unroll
-        for (int ob = 0; ob < 4; ob++) {
-            const int col = 16 * ob + 4 * g;
-            G[ob] = (ob < S::ob(LAYERS - 1) && valid && col < OUT) ? ld_h4(p.dy + (size_t)n * OUT + col) : h4zero();
-        }
-        dx_chain<IN, HID, OUT, LAYERS>(G, sfrag, p.fragT_off, p.acts, n, valid, lane);
-#pragma unroll
-        for (int ib = 0; ib < S::ib(0); ib++) {
-            const int col = 16 * ib + 4 * g;
-            if (valid && col < IN) st_h4(p.dx + (size_t)n * IN + col, G[ib]);
-        }
-    }
-}
-
 // grad[p] += sum over blocks of ws[b][p], summed in block order.
 struct ReduceParams {
     const float* ws;
@@ -545,43 +513,6 @@ void mlp_forward(const MlpShape& s, const FwdInput& in, const __half* const* W,
     }
 #undef GRAFT_FWD_LAUNCH
     GRAFT_LAUNCH_CHECK();
-}
-
-bool mlp_has_dx_kernel(const MlpShape& s)
-{
-    return s.in == 32 && s.hid == 64 && (s.out == 16 && s.layers == 2 || s.out == 8 && s.layers == 3);
-}
-
-bool mlp_backward_dx(const MlpShape& s, const __half* dy, const __half* const* acts, const __half* const* W,
-                     __half* dx, int N, hipStream_t stream, const uint32_t* d_n)
-{
-    s.validate();
-    if (!mlp_has_dx_kernel(s)) return false;
-    const bool density_head = s.out == 16;
-    if (dx == nullptr) throw std::runtime_error("TinyMLP: dX-only backward needs dx");
-    if (N <= 0) return true;
-    BwdParams p{};
-    p.dy = reinterpret_cast<const _Float16*>(dy);
-    p.acts = reinterpret_cast<const _Float16* const*>(acts);
-    p.W = reinterpret_cast<const _Float16* const*>(W);
-    p.dx = reinterpret_cast<_Float16*>(dx);
-    p.d_n = d_n;
-    p.N = N;
-    p.in = s.in;
-    p.hid = s.hid;
-    p.out_dim = s.out;
-    p.layers = s.layers;
-    int frag_halves = 0, unused = 0;
-    fill_layer_offsets(s, true, p.fragT_off, nullptr, frag_halves, unused);
-    const int lds = frag_halves * 2;
-    const auto kern = density_head ? mlp_bwd_dx_kernel<32, 64, 16, 2> : mlp_bwd_dx_kernel<32, 64, 8, 3>;
-    int per_cu = 0;
-    GRAFT_HIP_CHECK(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, 256, lds));
-    const int ntiles = (N + 15) / 16;
-    const int blocks = std::max(1, std::min((ntiles + 3) / 4, num_cus() * std::max(1, per_cu)));
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), lds, stream, p);
-    GRAFT_LAUNCH_CHECK();
-    return true;
 }
 
 void mlp_backward(const MlpShape& s, const __half* dy, const __half* const* acts,

@@ -942,7 +942,7 @@ def main():
                 "window": [prof_from, prof_from + len(prof_hits)], "mean_samples": round(n_prof, 1)}
     # MLP stages: the heads' forward (the encode is a stage of its own with the 16x16x32 heads), the dX
     # chains (main stream) and the weight gradients (side stream, beside the scatter)
-    mlp_ms = sum(st[k][0] for k in ("forward", "backwardDx", "colorDx", "densityDx", "colorBwd", "densityBwd",
+    mlp_ms = sum(st[k][0] for k in ("forward", "backwardDx", "colorBwd", "densityBwd",
                                     "headsBwd") if k in st)
     mfma_util = MLP_FLOP_PER_SAMPLE * n_prof / (mlp_ms * 1e-3) / 1e12 / FP16_PEAK_TFLOPS if mlp_ms else None
     mc = profile_json(MFMA_FILE)
