@@ -214,6 +214,7 @@ SIGNATURES = {
     "inerf_set_bg_color": (_i, [_vp, _f, _f, _f]),
     "inerf_set_step_limit": (_i, [_vp, _i]),
     "inerf_set_keep_color_dx": (_i, [_vp, _i]),
+    "inerf_set_keep_activations": (_i, [_vp, _i]),
     "inerf_last_rays_trained": (_u32, [_vp]),
     "inerf_set_profiling": (_i, [_vp, _i]),
     "inerf_print_stats": (_i, [_vp]),
@@ -542,6 +543,11 @@ class Nerf:
         """Keep each step's colour dL/d(input) in step_buffers().color_dx (introspection; the step
         with recomputed activations does not store it otherwise)."""
         self._c(self._L.inerf_set_keep_color_dx(self.h, int(on)))
+
+    def set_keep_activations(self, on):
+        """Later train() calls keep both heads' activations, the density head's 16 outputs and the whole
+        colour dL/d(input) in step_buffers() and the heads' buffers (introspection)."""
+        self._c(self._L.inerf_set_keep_activations(self.h, int(on)))
 
     def set_bg_color(self, r, g, b):
         self._c(self._L.inerf_set_bg_color(self.h, float(r), float(g), float(b)))

@@ -100,6 +100,7 @@ struct NerfBuffers {
     __half* color_dx = nullptr;
     __half* enc_planar = nullptr;    // [L][Bn] feature pairs: the step's encodings, level-major
     void* heads_packed = nullptr;    // both heads' weights packed for nerf_heads.hip (null: other shapes)
+    bool step_heads = false;         // the last step (before the first: the next one) ran nerf_heads.hip
     uint32_t* tile_live = nullptr;   // [Bn / 16 + 1]: 16-sample tiles with a nonzero gradient (dX -> dW)
     // occupancy
     float* tmp_grid = nullptr;
@@ -422,6 +423,7 @@ void InstantNerf::allocate()
     const graft::MlpShape csh = shape_of(cb.hw);
     if (graft::nerf_heads_supported(dsh, csh)) {
         b.heads_packed = dalloc<unsigned char>(graft::nerf_heads_packed_bytes());
+        b.step_heads = true;
         b.tile_live = dalloc<uint32_t>((size_t)Bn / 16 + 1);
         b.occ_packed = dalloc<unsigned char>(graft::nerf_heads_packed_bytes());
         b.occ_sorted = dalloc<float4>((size_t)b.occ_capacity);
@@ -469,6 +471,8 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
     const graft::MlpShape dshape{2 * o.numLevels, db.hw.hiddenDim, db.hw.outputDim, db.hw.numLayers};
     const graft::MlpShape cshape = shape_of(cb.hw);
     const int cstride = cb.hw.outputDim;
+    const bool heads = b.heads_packed != nullptr && !m_keepActivations;
+    b.step_heads = heads;
 
     auto stage_on = [&](hipStream_t s, const char* name, auto&& fn) {
         if (!o.isProfiling) {
@@ -579,7 +583,7 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
                                     cshape.layers},
             b.heads_packed, s);
     };
-    if (b.heads_packed) pack_heads(stream);
+    if (heads) pack_heads(stream);
     while (true) {
         StepSet& S = b.set[k];
         const uint32_t raysDone = S.raysDone;
@@ -620,7 +624,7 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
         };
         // hash encode (its own stage with the 16x16x32 heads), then density
         // head, SH gather and colour head
-        if (b.heads_packed)
+        if (heads)
             stage("encode", [&] {
                 graft::hash_encode_planar(b.meta, db.fwd_hashtable, reinterpret_cast<const float*>(S.positions), 4,
                                           b.enc_planar, (int)Bn, (int)Bn, stream, d_hits);
@@ -635,10 +639,10 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
             fa.dW = db.fwd_weights;
             fa.dB = db.master_biases;
             // the 16x16x32 heads store no activations: the backward recomputes them
-            fa.dacts = b.heads_packed ? nullptr : db.activations;
+            fa.dacts = heads ? nullptr : db.activations;
             fa.density_out = b.density_out;
             // the heads store the density logit 0 alone (all the step reads of it)
-            fa.density_stride = b.heads_packed ? 1 : 16;
+            fa.density_stride = heads ? 1 : 16;
             fa.dirs = cd;
             fa.ray_idx = S.ray_idx;
             fa.density_bias = o.densityBias;
@@ -647,14 +651,14 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
             fa.out_act = cb.hw.outputActivation;
             fa.cW = cb.fwd_weights;
             fa.cB = cb.master_biases;
-            fa.cacts = b.heads_packed ? nullptr : cb.activations;
+            fa.cacts = heads ? nullptr : cb.activations;
             fa.color_in = b.color_in;
             fa.color_out = cb.padded_outputs;
             fa.enc_scratch = b.enc_planar;
             fa.enc_plane = (int)Bn;
-            fa.heads_packed = b.heads_packed;
+            fa.heads_packed = heads ? b.heads_packed : nullptr;
             fa.heads_prepacked = true;  // packed at the call's start and after every step's layer Adam
-            fa.enc_ready = b.heads_packed != nullptr;
+            fa.enc_ready = heads;
             graft::nerf_forward(fa, (int)Bn, stream, d_hits);
         });
         // The next step's late refresh (one cascade): its samples are drawn
@@ -691,7 +695,7 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
             ga.offsets = S.offsets;
             ga.t = S.t_sorted;
             ga.density_out = b.density_out;
-            ga.density_stride = b.heads_packed ? 1 : 16;
+            ga.density_stride = heads ? 1 : 16;
             ga.color_out = cb.padded_outputs;
             ga.color_stride = cstride;
             ga.phi = b.phi;
@@ -723,7 +727,6 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
         hb.density_dy = db.dloss;
         hb.color_dx = m_keepColorDx ? b.color_dx : nullptr;  // read by nothing in the step
         hb.tile_live = b.tile_live;
-        const bool heads = b.heads_packed != nullptr;
         if (heads) {
             // recomputed activations: colour dX chain, glue, density dX chain
             stage("backwardDx", [&] { graft::nerf_heads_dx(hb, (int)Bn, stream, d_hits); });
@@ -840,7 +843,7 @@ void InstantNerf::trainWithRaysHit(const float3* d_rays_o, const float3* d_rays_
                 m_densityMLP->stepSplit(o.learningRate, o.beta1, o.beta2, o.epsilon, o.lossScale, b.side, stream);
             });
         // the next step's weights, packed beside this step's scatter
-        if (b.heads_packed) pack_heads(b.side);
+        if (heads) pack_heads(b.side);
         GRAFT_HIP_CHECK(hipEventRecord(b.ev_opt, b.side));
         opt_recorded = true;
 
@@ -1122,7 +1125,7 @@ InstantNerf::StepBuffers InstantNerf::stepBuffers() const
     s.ray_indices = S.ray_idx;
     s.t_sorted = S.t_sorted;
     s.density_out = b.density_out;
-    s.densityStride = b.heads_packed ? 1 : 16;
+    s.densityStride = b.step_heads ? 1 : 16;
     s.color_input = b.color_in;
     s.color_output = m_colorMLP->buffers().padded_outputs;
     s.sigma = b.sigma;
@@ -1138,7 +1141,7 @@ InstantNerf::StepBuffers InstantNerf::stepBuffers() const
     s.windowStart = m_windowStart;
     s.encodings = reinterpret_cast<half*>(b.enc_planar);
     s.encodingPlane = (uint32_t)std::max(1, m_opts.batchSize);
-    s.activationsSaved = b.heads_packed ? 0 : 1;
+    s.activationsSaved = b.step_heads ? 0 : 1;
     return s;
 }
 

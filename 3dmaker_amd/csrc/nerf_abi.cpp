@@ -653,6 +653,10 @@ int inerf_set_keep_color_dx(Inerf* h, int on)
 {
     return NERF_CALL("inerf_set_keep_color_dx", h->nerf.setKeepColorDx(on != 0));
 }
+int inerf_set_keep_activations(Inerf* h, int on)
+{
+    return NERF_CALL("inerf_set_keep_activations", h->nerf.setKeepActivations(on != 0));
+}
 int inerf_set_bg_color(Inerf* h, float r, float g, float b)
 {
     return NERF_CALL("inerf_set_bg_color", h->nerf.setBgColor(make_float3(r, g, b)));

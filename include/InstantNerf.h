@@ -127,6 +127,12 @@ public:
     // on (off by default); the other path always stores it (its density
     // gradient glue reads it).
     void setKeepColorDx(bool keep) { m_keepColorDx = keep; }
+    // Addition (introspection): keep what the 16x16x32 heads' step does not
+    // store, for the calls that follow (off by default).  The step then runs
+    // the kernels of the other head shapes: stepBuffers() reports
+    // activationsSaved 1 and a density stride of 16, both heads' activation
+    // buffers hold the step's, color_dx all 32 columns, and no tile is skipped.
+    void setKeepActivations(bool keep) { m_keepActivations = keep; }
 
     // InstantNerf.cu:359-583.  d_rays_depth / d_rays_sigma may be null (depth
     // supervision off), d_rgb_true must be set, hitCounts (host, nullable)
@@ -231,6 +237,7 @@ private:
     int m_stepLimit = 0;
     uint32_t m_lastRaysTrained = 0;
     bool m_keepColorDx = false;
+    bool m_keepActivations = false;
 
     uint8_t* d_occupancyGrid = nullptr;
     size_t m_occupancyBytes = 0;

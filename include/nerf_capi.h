@@ -97,6 +97,10 @@ uint32_t inerf_last_rays_trained(Inerf* h);
  * color_dx, which the step with recomputed activations otherwise does not
  * store. */
 int inerf_set_keep_color_dx(Inerf* h, int on);
+/* InstantNerf::setKeepActivations (no reference counterpart; introspection):
+ * on != 0 has the steps of later inerf_train calls keep both heads'
+ * activations, the density head's 16 outputs and the whole color_dx. */
+int inerf_set_keep_activations(Inerf* h, int on);
 int inerf_set_profiling(Inerf* h, int on);
 int inerf_print_stats(Inerf* h);
 /* Per-stage profiling means as "stage:mean_ms:calls;..." into buf (NUL-terminated,

@@ -1,5 +1,6 @@
-"""Training steps with the colour heads INerfTrainer (32 x 3) and InstantNerf's defaults (64 x 2) use, and the smallest
-one (32 x 2), replayed stage by stage on the oracle from the GPU's state before each step."""
+"""Training steps with the colour heads INerfTrainer (32 x 3) and InstantNerf's defaults (64 x 2) use, the smallest
+one (32 x 2) and one outside the 16x16x32 heads (64 x 4), replayed stage by stage on the oracle from the GPU's state
+before each step; with the activations kept on request, and with the request turned on between two calls."""
 import os
 import sys
 
@@ -19,9 +20,11 @@ scenes = importlib.import_module("3dmaker_amd.scenes")
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("hidden,layers", [(32, 3), (64, 2), (32, 2)])
-def test_steps_match_oracle(hidden, layers):
-    print(f"[head shape] {hidden} x {layers}", flush=True)
+@pytest.mark.parametrize("hidden,layers,keep", [(32, 3, 0), (64, 2, 0), (32, 2, 0), (64, 4, 0), (32, 3, 1), (64, 2, 1),
+                                                (32, 2, 1), (64, 3, 1), (32, 3, 2)])
+def test_steps_match_oracle(hidden, layers, keep):
+    """keep: 1 the activations from the first step on, 2 from the second."""
+    print(f"[head shape] {hidden} x {layers} keep={keep}", flush=True)
     P = pkg()
     o = P.Nerf.default_options()
     o.gridResolution[:] = [32, 32, 32]
@@ -39,7 +42,9 @@ def test_steps_match_oracle(hidden, layers):
     nerf.set_learning_rate(lr)
     nerf.set_bg_color(*bg)
     first = 0
-    for _ in range(3):
+    for step in range(3):
+        if keep and step == keep - 1:
+            nerf.set_keep_activations(True)
         st = nc.read_state(nerf, o)
         march = nc.oracle_active(o, st, ro[first:], rd[first:])
         R = int(march["active"])
@@ -50,6 +55,9 @@ def test_steps_match_oracle(hidden, layers):
         n, hits = nerf.train(dev[0], dev[1], dev[2], R, rgb_out=rgb)
         torch.cuda.synchronize()
         assert n == 1 and int(hits[0]) == int(march["total"])
+        b = nerf.step_buffers()
+        kept = layers == 4 or (keep and step >= keep - 1)
+        assert (b.activationsSaved, b.density_stride) == ((1, 16) if kept else (0, 1))
         nc.check_step(nerf, o, st, march, ro[sl], rd[sl], gt[sl], R, bg, lr, rgb.cpu().numpy())
         first += R
     nerf.close()
