@@ -1371,8 +1371,9 @@ namespace {
 // other, a chain of LDS atomics per level, so a small batch (few rounds) is
 // bound by that chain and cuts the levels over enough workgroups for one per
 // CU: a training step of 4096 points 103 -> 75 us (with the single accumulate
-// launch below); with 8 or 4 levels per workgroup instead of one 87 and 81.  From
-// 256 rounds on the GPU is full and a round keeps all its levels: with two
+// launch below); with 8 or 4 levels per workgroup instead of one 87 and 81.  The
+// groups fill at most one workgroup per CU: two from 86 to 128 rounds, and from
+// 129 rounds on (65,537 samples) a round keeps all its levels.  With two
 // groups at 2^18 samples every row of dL/denc is fetched twice, a training
 // step over rays 3 % slower, a stand-alone scatter of ray samples 4 % faster.
 int level_groups(ScatterArgs& a)

@@ -12,9 +12,16 @@ from helpers import pkg
 
 torch = pytest.importorskip("torch")
 
+BELOW_ONE = float(np.nextafter(np.float32(1), np.float32(0)))
 BOXES = [([-1.5] * 3, [1.5] * 3), ([-0.7] * 3, [0.7] * 3), ([-1.3] * 3, [1.3] * 3), ([-11.9] * 3, [11.9] * 3),
-         ([-0.9999999] * 3, [0.9999999] * 3),            # an extent with an all-ones significand: divides
-         ([-1.3, -1.3, -1.3], [1.3, 1.3, 1.4]), ([-1.0, -1.2, -1.1], [1.1, 1.0, 1.2])]
+         ([-0.9999999] * 3, [0.9999999] * 3),
+         ([-1.3, -1.3, -1.3], [1.3, 1.3, 1.4]), ([-1.0, -1.2, -1.1], [1.1, 1.0, 1.2]),
+         ([-BELOW_ONE] * 3, [BELOW_ONE] * 3)]             # an extent with an all-ones significand: divides
+
+
+def test_the_last_box_has_an_all_ones_extent():
+    mn, mx = (np.float32(v[0]) for v in BOXES[-1])
+    assert (mx - mn).view(np.uint32) & 0x7fffff == 0x7fffff
 
 
 def fma32(a, b, c):

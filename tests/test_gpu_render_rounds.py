@@ -1,6 +1,7 @@
-"""The front-to-back render against one whole-ray evaluation of the same rays: samples by the march launcher, the
-heads' own kernels and the oracle's inference compositing.  Rays with one to hundreds of samples, thin and opaque
-fields, chunks of rays larger than a hit batch holds, none, one and odd ray counts."""
+"""Renders of both forms against the oracle's march, heads and inference compositing of the same rays.  Front to back in
+rounds: rays with one to hundreds of samples, thin and opaque fields, chunks of rays larger than a hit batch holds, one
+and odd ray counts, boxes that are no cube.  Whole rays: several ray chunks, several hit batches per chunk, several
+samples per voxel.  A ray's colour has the same bits in both."""
 import os
 import sys
 
@@ -29,16 +30,34 @@ pytestmark = pytest.mark.gpu
     (777, 1 << 12, 3, 1.0, 64, 4),      # cascades; a colour head outside the MFMA kernels' shapes
 ])
 def test_render_matches_whole_rays(R, batch, cascades, bias, hidden, layers):
-    print(f"[render rounds] R={R} batch={batch} C={cascades} bias={bias} colour {hidden} x {layers}", flush=True)
+    check(R, batch, cascades, bias, hidden, layers)
+
+
+@pytest.mark.parametrize("R,K", [(900, 1), (3000, 2), (700, 3)])
+def test_whole_rays_in_chunks_and_hit_batches(R, K):
+    """R <= hit batch / 20, or several samples per voxel: whole rays, here of several chunks of 256 rays."""
+    batch = 20 * R if K == 1 else 1 << 12
+    N = check(R, batch + 16, 1, 0.0, 64, 2, K=K, chunk=256)
+    assert K == 1 or N > 3 * batch        # several hit batches
+
+
+@pytest.mark.parametrize("mn,mx,cascades", [((-1.3, -1.5, -1.4), (1.4, 1.5, 1.2), 1), ((-1.5,) * 3, (1.5, 1.5, 1.75), 3)])
+def test_rounds_in_a_box_that_is_no_cube(mn, mx, cascades):
+    check(2047, 1 << 14, cascades, 1.0, 64, 3, mn=mn, mx=mx)
+
+
+def check(R, batch, cascades, bias, hidden, layers, K=1, chunk=1024, mn=(-1.5,) * 3, mx=(1.5,) * 3):
+    print(f"[render rounds] R={R} batch={batch} C={cascades} bias={bias} colour {hidden} x {layers} "
+          f"K={K} chunk={chunk} box {mn} {mx}", flush=True)
     P = pkg()
     res, mips, T_ = 64, 4, 1 << 14
     o = P.Nerf.default_options()
     o.gridResolution[:] = [res] * 3
-    o.aabbMin[:], o.aabbMax[:] = [-1.5] * 3, [1.5] * 3
-    o.levelsMipmap, o.numCascades, o.samplesPerVoxel = mips, cascades, 1
+    o.aabbMin[:], o.aabbMax[:] = mn, mx
+    o.levelsMipmap, o.numCascades, o.samplesPerVoxel = mips, cascades, K
     o.hashTableSize, o.growthFactor = T_, 1.447
     o.colorHiddenDim, o.colorNumLayers = hidden, layers
-    o.batchSize, o.rayChunkSize, o.renderBatchSize = batch, 1024, batch
+    o.batchSize, o.rayChunkSize, o.renderBatchSize = batch, chunk, batch
     o.densityBias = bias
     o.bgColor[:] = [0.25, 0.5, 1.0]
     nerf = P.Nerf(o)
@@ -58,9 +77,9 @@ def test_render_matches_whole_rays(R, batch, cascades, bias, hidden, layers):
     torch.cuda.synchronize()
     np.testing.assert_array_equal(rgb.cpu().numpy(), rgb2.cpu().numpy())
 
-    mn, mx = np.float32([-1.5] * 3), np.float32([1.5] * 3)
+    mn, mx = np.float32(mn), np.float32(mx)
     di, near, far = orc.ray_aabb_inv(ro, rd, mn, mx, cascades)
-    m = orc.march_hits(ro, rd, di, near, far, bits, [res] * 3, mn, mx, cascades, mips, 1, 1 << 24)
+    m = orc.march_hits(ro, rd, di, near, far, bits, [res] * 3, mn, mx, cascades, mips, K, 1 << 24)
     N = int(m["total"])
     cnt, off, t, ridx = m["counts"][:R], m["offsets"][:R], m["t"][:N], m["ray_idx"][:N]
     assert N > 0 or R == 1
@@ -82,6 +101,7 @@ def test_render_matches_whole_rays(R, batch, cascades, bias, hidden, layers):
     if cascades == 1 and R > 1:
         assert cnt.max() > 17  # more than one round
     nerf.close()
+    return N
 
 
 @pytest.mark.parametrize("hidden,layers", [(32, 3), (64, 2), (64, 4)])   # the last one outside the MFMA heads

@@ -1,5 +1,5 @@
 """The table-gradient scatter where its launches change: level groups per batch size (one level per workgroup
-for the smallest, all levels from 256 rounds of 512 samples on), the largest batch without a second accumulate
+for the smallest, 4 at 85 rounds of 512 samples, 8 from 86 to 128, all levels from 129 on), the largest batch without a second accumulate
 launch and the next one, level counts that leave a short last group, and gradients off 16-byte alignment; within
 the per-word bound of the oracle's fp64 sums."""
 import numpy as np
@@ -16,7 +16,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("N,L,shift,spread", [(1, 16, 0, 1.0), (511, 7, 0, 1.0), (513, 17, 2, 1.0), (4096, 16, 0, 1e-3),
                                               (6144, 16, 0, 1e-3), (6145, 16, 2, 1e-3), (8192, 5, 0, 1e-3),
-                                              (8193, 16, 0, 1e-3), (33333, 12, 2, 1.0), (65537, 9, 0, 0.1),
+                                              (8193, 16, 0, 1e-3), (33333, 12, 2, 1.0), (85 * 512, 16, 0, 0.1),
+                                              (85 * 512 + 1, 16, 0, 0.1), (65536, 16, 2, 0.1), (65537, 16, 0, 0.1),
+                                              (65536, 20, 0, 1.0), (65537, 9, 0, 0.1),
                                               (130560, 16, 2, 1.0), (130561, 16, 0, 0.1)])
 def test_scatter_groups_match_oracle(N, L, shift, spread):
     P = pkg()
