@@ -34,9 +34,10 @@ GRAFT_HD int row_base(int hid, int in, int l)
 // matrix) and goes to half dst.  Every layer behind layer 0 has hid rows but
 // the last, which may have more.  Rows of both kinds are 8 halves apart from
 // each other, so that dst is q and the rows before it.  Written for few
-// instructions, one chunk per thread: what a small batch waits for (1,003
-// samples of 8-128-128-128-8 11.3 to 11.8 us with rows and columns
-// worked out apart, 10.8 so).
+// instructions and no branch, one chunk per thread: what a small batch waits
+// for (1,003 samples of 8-128-128-128-8 11.3 to 11.8 us with rows and columns
+// worked out apart, 10.8 with the two kinds of rows in branches, 10.2 so;
+// 3,001 of 32-32-16 5.8 and 5.3).
 struct Staged {
     int layer, at, dst;
     bool ok;
@@ -49,16 +50,16 @@ GRAFT_HD Staged staged_chunk(int q, int hid, int in, int out, int layers)
 {
     const int blocks = up32(in) / 32, first_end = hid * blocks * 4;  // a row of layer 0 has 4 * blocks chunks
     const int reciprocal = blocks == 1 ? 65536 : blocks == 2 ? 32768 : blocks == 3 ? 21846 : 16384;  // of blocks, 2^16
-    const bool first = q < first_end;
+    const int first = q < first_end ? -1 : 0;  // all bits: both sides are worked out and selected, without a branch
     const int row0 = ((q >> 2) * reciprocal) >> 16;
     const int R = (q - first_end) >> (hid == 128 ? 4 : hid == 64 ? 3 : 2);  // row behind layer 0 (negative: layer 0)
     const int piece = R >> (hid == 128 ? 7 : hid == 64 ? 6 : 5);
     const int l = piece < -1 ? 0 : piece > layers - 2 ? layers - 1 : piece + 1;
     Staged s;
     s.layer = l;
-    s.dst = 8 * (q + (first ? row0 : hid + R));
-    s.at = 8 * q + (first ? row0 * (in - 32 * blocks) : -8 * first_end - (l - 1) * hid * hid);
-    s.ok = first ? 8 * q - row0 * 32 * blocks < in : R < (layers - 2) * hid + out;
+    s.dst = 8 * (q + ((row0 & first) | ((hid + R) & ~first)));
+    s.at = 8 * q + ((row0 * (in - 32 * blocks) & first) | ((-8 * first_end - (l - 1) * hid * hid) & ~first));
+    s.ok = (((8 * q - row0 * 32 * blocks) & first) | (R & ~first)) < ((in & first) | (((layers - 2) * hid + out) & ~first));
     return s;
 }
 
