@@ -36,8 +36,7 @@ GRAFT_HD int row_base(int hid, int in, int l)
 // each other, so that dst is q and the rows before it.  Written for few
 // instructions and no branch, one chunk per thread: what a small batch waits
 // for (1,003 samples of 8-128-128-128-8 11.3 to 11.8 us with rows and columns
-// worked out apart, 10.8 with the two kinds of rows in branches, 10.2 so;
-// 3,001 of 32-32-16 5.8 and 5.3).
+// worked out apart, 10.8 with the two kinds of rows in branches, 10.2 so).
 struct Staged {
     int layer, at, dst;
     bool ok;
