@@ -1231,7 +1231,7 @@ uint32_t InstantNerf::renderHitBatch() const
 // lie behind saturation; the rounds, whose rays march and evaluate 8 to 32 samples
 // before they are asked, evaluate 7.6 M.
 // With several samples per voxel (a round ends between voxels), without an
-// output or with few rays, whole rays per hit batch: compaction from the first unrendered ray,
+// output, with few rays or a small hit batch, whole rays per hit batch: compaction from the first unrendered ray,
 // one host read per hit batch; the reference makes three blocking ones.  Both
 // forms run the same encode and head kernels and the same compositing
 // operations, so that a ray's colour does not depend on the rays beside it

@@ -71,17 +71,23 @@ constexpr int kSegmentRounds = kMaxHits / kSegmentLeast + 2;
 constexpr uint32_t kSegmentLast = 0x80000000u;  // in count: no sample behind this round's
 // Whether a render of R rays goes in rounds.  A round costs at least its
 // launches, about 40 us, and one more runs before the host knows that no ray
-// is left; few rays that go into a hit batch or two (20 samples a ray) are
+// is left: it takes a hit batch of kSegmentBatch for a round's work to outweigh
+// that, and few rays that go into a hit batch or two (20 samples a ray) are
 // faster as whole rays.
-// Whole rays against rounds in us, hit batch 2^21: 120 x 90 rays 218 / 256,
-// 160 x 120 264 / 289, 180 x 135 293 / 310 (292 / 289 in another scene), 200 x
-// 150 324 / 330 (319 / 306), 256 x 192 431 / 402, 320 x 240 737 / 484; hit batch
-// 2^18: 100 x 75 198 / 246, 120 x 90 279 / 259 (two hit batches), 140 x 105
-// 301 / 312, 160 x 120 388 / 343, 201 x 151 512 / 368.
+// Whole rays against rounds in us.  400 x 300 rays, nine scenes, hit batch 2^16:
+// 2,188 / 3,308 (1,868 / 3,011 where least lies behind saturation, 8,285 / 5,365
+// where most does); 2^17: 1,684 / 1,858 (1,218 / 1,773, 5,050 / 3,286); 2^18:
+// 1,190 / 1,298 (867 / 1,006, 3,277 / 2,024), six of the nine faster in rounds;
+// 2^21, two scenes: 968 / 702 and 1,009 / 652.  Hit batch 2^21: 120 x 90 rays
+// 218 / 256, 160 x 120 264 / 289, 180 x 135 293 / 310 (292 / 289 in another
+// scene), 200 x 150 324 / 330 (319 / 306), 256 x 192 431 / 402, 320 x 240 737 /
+// 484; hit batch 2^18: 100 x 75 198 / 246, 120 x 90 279 / 259 (two hit batches),
+// 140 x 105 301 / 312, 160 x 120 388 / 343, 201 x 151 512 / 368.
 constexpr uint32_t kSegmentRays = 24576;
+constexpr uint32_t kSegmentBatch = 1u << 18;
 constexpr bool render_in_rounds(uint32_t R, uint32_t hit_batch)
 {
-    return R >= kSegmentRays || R > hit_batch / 20u;
+    return hit_batch >= kSegmentBatch && (R >= kSegmentRays || R > hit_batch / 20u);
 }
 struct RenderSegments {
     // per ray

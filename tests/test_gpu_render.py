@@ -1,9 +1,9 @@
 """GPU parity of the inference render path and the model queries against the oracle.
 
 renderImageHit (InstantNerf.cu:713-864) runs density inference, SH gather, colour
-inference and the inference compositor (compositing.cu:5-78): many rays front to
-back in rounds of samples, few rays (or several samples per voxel) whole, a hit
-batch at a time.  Bars: the compositor is
+inference and the inference compositor (compositing.cu:5-78): many rays with a
+large hit batch front to back in rounds of samples, the others whole, a hit batch
+at a time.  Bars: the compositor is
 bit-exact on identical inputs; a rendered colour is within 2e-3 abs / 1e-2 rel
 of the oracle chain (fp16 MLP operands, fp32 accumulation in another order);
 a ray's colour does not depend on how rays are split into chunks and hit
@@ -120,9 +120,9 @@ def test_inference_compositor_bit_exact(dev):
 
 
 def test_render_matches_oracle_chain(dev):
-    """Rounds over several chunks of rays (a chunk is an eighth of the hit batch); colour vs
-    the oracle chain, and identical bits with a larger INFERENCE hit batch.  (Whole rays in
-    chunks and hit batches: test_gpu_render_rounds.py.)"""
+    """Several ray chunks and several hit batches per chunk; colour vs the oracle
+    chain, and identical bits with a larger INFERENCE hit batch.  (Rounds, and both
+    forms against each other: test_gpu_render_rounds.py.)"""
     P = pkg()
     nerf = P.Nerf(options(P, batch=2048, chunk=704, render_batch=1 << 15))
     bits = grid_bits(13)

@@ -22,12 +22,18 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("R,batch,cascades,bias,hidden,layers", [
-    (1, 1 << 14, 1, 0.0, 64, 3),        # one ray
-    (819, 1 << 14, 1, 0.0, 64, 3),      # the most rays that go whole at this hit batch, and one more
+    (1, 1 << 14, 1, 0.0, 64, 3),        # whole rays: a hit batch below 2^18.  One ray
+    (819, 1 << 14, 1, 0.0, 64, 3),
     (820, 1 << 14, 1, 0.0, 64, 3),
-    (2047, 1 << 14, 1, 4.0, 32, 3),     # thin field: no ray saturates, many rounds
-    (5000, 1 << 14, 1, -6.0, 64, 2),    # opaque field: most rays end in the first round; several chunks of rays
+    (2047, 1 << 14, 1, 4.0, 32, 3),     # thin field: no ray saturates
+    (5000, 1 << 14, 1, -6.0, 64, 2),    # opaque field
     (777, 1 << 12, 3, 1.0, 64, 4),      # cascades; a colour head outside the MFMA kernels' shapes
+    (13107, 1 << 18, 1, 0.0, 64, 3),    # the most rays that go whole at this hit batch, and one more, in rounds
+    (13108, 1 << 18, 1, 0.0, 64, 3),
+    (13107, (1 << 18) - 16, 1, 0.0, 32, 2),  # a hit batch below the rounds'
+    (14001, 1 << 18, 1, 4.0, 32, 3),    # rounds.  Thin field: no ray saturates, many rounds
+    (40001, 1 << 18, 1, -6.0, 64, 2),   # opaque field: most rays end in the first round; two chunks of rays
+    (15001, 1 << 18, 3, 1.0, 64, 4),    # cascades; a colour head outside the MFMA kernels' shapes
 ])
 def test_render_matches_whole_rays(R, batch, cascades, bias, hidden, layers):
     check(R, batch, cascades, bias, hidden, layers)
@@ -35,7 +41,7 @@ def test_render_matches_whole_rays(R, batch, cascades, bias, hidden, layers):
 
 @pytest.mark.parametrize("R,K", [(900, 1), (3000, 2), (700, 3)])
 def test_whole_rays_in_chunks_and_hit_batches(R, K):
-    """R <= hit batch / 20, or several samples per voxel: whole rays, here of several chunks of 256 rays."""
+    """One and several samples per voxel: whole rays, here of several chunks of 256 rays."""
     batch = 20 * R if K == 1 else 1 << 12
     N = check(R, batch + 16, 1, 0.0, 64, 2, K=K, chunk=256)
     assert K == 1 or N > 3 * batch        # several hit batches
@@ -43,7 +49,7 @@ def test_whole_rays_in_chunks_and_hit_batches(R, K):
 
 @pytest.mark.parametrize("mn,mx,cascades", [((-1.3, -1.5, -1.4), (1.4, 1.5, 1.2), 1), ((-1.5,) * 3, (1.5, 1.5, 1.75), 3)])
 def test_rounds_in_a_box_that_is_no_cube(mn, mx, cascades):
-    check(2047, 1 << 14, cascades, 1.0, 64, 3, mn=mn, mx=mx)
+    check(14003, 1 << 18, cascades, 1.0, 64, 3, mn=mn, mx=mx)
 
 
 def check(R, batch, cascades, bias, hidden, layers, K=1, chunk=1024, mn=(-1.5,) * 3, mx=(1.5,) * 3):
@@ -109,7 +115,7 @@ def test_a_ray_has_one_colour_however_rays_are_grouped(hidden, layers):
     """The same rays in one call (rounds), in calls small enough to go whole, alone, and with another hit batch: the
     same bits."""
     P = pkg()
-    res, mips, T_, R, batch = 64, 4, 1 << 14, 3000, 1 << 14
+    res, mips, T_, R, batch = 64, 4, 1 << 14, 16000, 1 << 18
     small = batch // 20                  # the most rays that go whole
     o = P.Nerf.default_options()
     o.gridResolution[:] = [res] * 3
@@ -117,7 +123,7 @@ def test_a_ray_has_one_colour_however_rays_are_grouped(hidden, layers):
     o.levelsMipmap, o.numCascades, o.samplesPerVoxel = mips, 1, 1
     o.hashTableSize, o.growthFactor = T_, 1.447
     o.colorHiddenDim, o.colorNumLayers = hidden, layers
-    o.batchSize, o.rayChunkSize, o.renderBatchSize = batch, 512, 1 << 16
+    o.batchSize, o.rayChunkSize, o.renderBatchSize = batch, 512, 1 << 19
     nerf = P.Nerf(o)
     rng = np.random.default_rng(3)
     nerf.density.load_hashgrid(rng.normal(0, 0.5, 16 * T_ * 2).astype(np.float32))
@@ -135,7 +141,7 @@ def test_a_ray_has_one_colour_however_rays_are_grouped(hidden, layers):
     whole = render([0, R])
     assert len(np.unique(whole[:, 0])) > R // 2   # colours, not the background
     np.testing.assert_array_equal(render(list(range(0, R, small)) + [R]), whole)
-    np.testing.assert_array_equal(render([0, 1, 2, 17, small + 17, R]), whole)
-    nerf.set_memory_mode(True)                    # a hit batch of 2^16: R <= 2^16 / 20 goes whole
+    np.testing.assert_array_equal(render([0, 1, 2, 17, 3000, R]), whole)
+    nerf.set_memory_mode(True)                    # a hit batch of 2^19: R <= 2^19 / 20 goes whole
     np.testing.assert_array_equal(render([0, R]), whole)
     nerf.close()
