@@ -154,7 +154,7 @@ struct Fwd32Params {
 // saved activations and outputs for wide batches; the loads of the next tiles
 // are issued before the current ones are computed.
 // 2^18 samples through 64-64-64-64-64 with saved activations, 168 MB written and 34 read: 104 us and a 23 us copy to
-// the caller's rows before, 65 us with that copy in it.
+// the caller's rows before, 58 us with that copy in it.
 template <int HB, int NT, int MODE, bool SAVE, int OUT_ACT>
 __global__ __launch_bounds__(256) void mlp32_fwd_kernel(const Fwd32Params p)
 {
@@ -436,7 +436,7 @@ __device__ __forceinline__ h8 lds_tr8(const _Float16* p, int pitch)
 // What is left is the bytes of dL/dy and activations (33 us for 2^18 samples
 // of 64-64-64-64-64 at a large copy's rate) and two barriers per layer: 76 us,
 // 150 with 2-byte transposing LDS writes and 16x16x16 products before; 65,537
-// samples of 32-64-64-8 21 us, 37 before; 2^18 of 32-64-16 32 us, 33 before.
+// samples of 32-64-64-8 20 us, 37 before; 2^18 of 32-64-16 28 us, 33 before.
 template <int HB, int LAYERS>
 __global__ __launch_bounds__(256, HB == 1 ? 4 : HB == 2 ? 2 : 1) void mlp32_bwd_kernel(const Bwd32Params p)
 {
