@@ -135,7 +135,8 @@ struct NerfBuffers {
         __half* color_in = nullptr;    // [cap x 32]
         float* sigma = nullptr;
         float* rgb = nullptr;          // [cap x colour head width] (padded)
-        __half* enc = nullptr;         // [cap x 2L] level-major encodings of a hit batch or round
+        __half* enc = nullptr;         // [enc_cap x 2L] level-major encodings of a hit batch or round
+        uint32_t enc_cap = 0;
         uint32_t rays = 0;             // rays of one chunk of the rounds
         graft::RenderSegments seg{};   // per ray of a chunk, and the rounds' counters
         uint32_t* h_live = nullptr;    // pinned [kSegmentRounds + 1]: live rays after each round
@@ -1159,7 +1160,6 @@ void ensure_render(NerfBuffers& b, uint32_t cap, int color_width)
     dfree(b.render.color_in);
     dfree(b.render.sigma);
     dfree(b.render.rgb);
-    dfree(b.render.enc);
     b.render.cap = 0;
     b.render.positions = dalloc<float4>(cap);
     b.render.ray_idx = dalloc<uint32_t>(cap);
@@ -1168,8 +1168,17 @@ void ensure_render(NerfBuffers& b, uint32_t cap, int color_width)
     b.render.color_in = dalloc<__half>((size_t)cap * 32);
     b.render.sigma = dalloc<float>(cap);
     b.render.rgb = dalloc<float>((size_t)cap * color_width);
-    b.render.enc = dalloc<__half>((size_t)2 * b.meta.numLevels * cap);
     b.render.cap = cap;
+}
+
+// Room for the encodings of a hit batch: renders alone need it, not the queries.
+void ensure_encodings(NerfBuffers& b, uint32_t cap)
+{
+    if (b.render.enc_cap >= cap) return;
+    dfree(b.render.enc);
+    b.render.enc_cap = 0;
+    b.render.enc = dalloc<__half>((size_t)2 * b.meta.numLevels * cap);
+    b.render.enc_cap = cap;
 }
 
 // What a front-to-back render of the hit batch `cap` keeps, on first use and
@@ -1249,6 +1258,7 @@ void InstantNerf::renderImageHit(const float3* d_rays_o, const float3* d_rays_d,
     const graft::MlpShape dshape{2 * o.numLevels, db.hw.hiddenDim, db.hw.outputDim, db.hw.numLayers};
     const graft::MlpShape cshape = shape_of(cb.hw);
     ensure_render(b, hitBatch, cshape.out);
+    ensure_encodings(b, hitBatch);
     // a render discards the prefetched rays; its whole-ray form also reuses the march store and step set 0
     b.ms[0].version = b.ms[1].version = -1;
     b.pre.valid = false;
